@@ -126,7 +126,9 @@ int thv_graph_info(const thv_graph *g, uint64_t *n, uint64_t *m,
  *                       0: top-down only, as in the reference
  *   THV_OPT_DO_ALPHA    all edges in HBM: top-down -> bottom-up when
  *                       frontier edges exceed unvisited edges / alpha
- *                       (default 14)
+ *                       (default 14; until a caller sets it, a frontier of
+ *                       at most 4,096 vertices and 32,768 edges stays
+ *                       top-down)
  *   THV_OPT_DO_BETA     all edges in HBM: bottom-up -> top-down when the
  *                       frontier holds fewer than n / beta vertices (24)
  *   THV_OPT_DO_VERTEX_NS  split store: a level runs bottom-up when its

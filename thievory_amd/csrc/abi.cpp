@@ -108,6 +108,7 @@ int thv_graph_set_option(thv_graph *gh, int option, double value) {
       case THV_OPT_DO_ALPHA:
         NEED(value > 0.0);
         g->do_alpha = value;
+        g->do_alpha_set = true;
         break;
       case THV_OPT_DO_BETA:
         NEED(value > 0.0);

@@ -230,10 +230,121 @@ static ExpandArgs base_args(Graph &g, Workspace &w) {
 }
 static ExpandArgs base_args(Graph &g) { return base_args(g, g.ws); }
 
+constexpr int AUX_COUNT = 14;  // aux[14]: the listed frontier's size (0 between launches)
+constexpr int AUX_SMALL = 16;  // aux / h_aux[16, 28): SmallOut
+static_assert(AUX_SMALL + sizeof(SmallOut) / 8 <= AUX_WORDS, "SmallOut fits the counters");
+
+// Whether a frontier of these vertices and edges is worth handing to
+// k_small: what it takes itself.
+static bool small_frontier(uint64_t nf, uint64_t mf, Algo algo = A_BFS) {
+  return nf <= SPARSE_MAX && mf <= (algo == A_SSSP ? SMALL_EDGES_SSSP : SMALL_EDGES);
+}
+
+// Levels from the frontier {src} (from_src: its bit alone is set in
+// `front`) or from the one the bitmap holds, run by k_small until the
+// frontier is empty or too large; returns after the stream has drained.
+// The levels' counts go to st, the kernel's time (with events) to *ms.
+// edge_max, ratio, unvisited: when a BFS is handed back for its direction to
+// be chosen (SmallArgs).  side (listed frontiers, may be null): words the
+// listing clears.
+static SmallOut run_small(Graph &g, Workspace &w, Algo algo, uint32_t *front, bool from_src,
+                          uint32_t src, uint32_t level_value, uint32_t thr, uint32_t delta,
+                          bool timed, double *ms, thv_stats *st,
+                          uint64_t edge_max = SMALL_EDGES, double ratio = 0,
+                          uint64_t unvisited = 0, const LevelSide *side = nullptr) {
+  hipStream_t s = g.stream;
+  QueueSet &q = w.qs;
+  SmallArgs a;
+  memset(&a, 0, sizeof a);
+  a.deg = g.d_deg.as<uint32_t>();
+  a.rbit = g.store.d_rbit.as<uint32_t>();
+  a.vpart = g.store.d_vpart.as<uint32_t>();
+  a.pres = g.store.d_pres.as<uint8_t>();
+  a.eptr = g.store.d_eptr.as<uint64_t>();
+  a.ptouch = q.ptouch.as<uint32_t>();
+  if (q.stamp > 0xFFFFFFFFu - SMALL_LEVELS - 2) {  // would wrap: old stamps could collide
+    launch_fill_u32(a.ptouch, 0u, (uint64_t)q.P + 1, s);
+    q.stamp = 0;
+  }
+  a.stamp = q.stamp + 1;
+  a.split = g.store.host_vertices > 0 || g.store.Pdev < g.store.P;
+  a.val = w.val.as<uint32_t>();
+  a.vis = w.vis.as<uint32_t>();
+  a.front = front;
+  unsigned long long *aux = w.aux.as<unsigned long long>();
+  // the general path's queue arrays are free between its levels
+  a.far[0] = q.qe[0].as<unsigned long long>();
+  a.far[1] = q.qe[1].as<unsigned long long>();
+  a.far_cap = (uint32_t)std::min<uint64_t>(g.n + 1, 1u << 16);
+  a.src = src;
+  a.level_value = level_value;
+  a.thr = thr;
+  a.delta = delta;
+  a.edge_max = (uint32_t)std::min<uint64_t>(
+      edge_max, algo == A_SSSP ? SMALL_EDGES_SSSP : SMALL_EDGES);
+  a.ratio = ratio;
+  a.unvisited = unvisited;
+  a.max_levels = SMALL_LEVELS;
+  const bool mapped = w.h_aux_dev != nullptr;
+  a.out = reinterpret_cast<SmallOut *>((mapped ? w.h_aux_dev : aux) + AUX_SMALL);
+  if (!from_src) {
+    a.list = q.qv[0].as<uint32_t>();
+    a.count = reinterpret_cast<unsigned int *>(aux + AUX_COUNT);
+    const uint32_t cap = algo == A_SSSP ? a.far_cap : SPARSE_MAX;
+    launch_list_front(g, front, q.qv[0].as<uint32_t>(), (uint32_t)std::min<uint64_t>(cap, g.n),
+                      a.count, s, side);
+  }
+  if (timed) HIPC(hipEventRecord(w.ev[0], s));
+  launch_small(g, algo, a, s);
+  if (timed) HIPC(hipEventRecord(w.ev[1], s));
+  SmallOut o;
+  if (!mapped) HIPC(hipMemcpyAsync(&o, a.out, sizeof o, hipMemcpyDeviceToHost, s));
+  HIPC(hipStreamSynchronize(s));
+  if (mapped) memcpy(&o, w.h_aux + AUX_SMALL, sizeof o);
+  q.stamp += (uint32_t)o.levels + 1;
+  if (timed) {
+    float t = 0;
+    HIPC(hipEventElapsedTime(&t, w.ev[0], w.ev[1]));
+    *ms += t;
+  }
+  if (st) {
+    const uint64_t rec = (uint64_t)g.rec, e = o.edges[0] + o.edges[1];
+    const uint64_t hbm = o.edges[1] * rec + 4 * e + 12 * o.vertices;
+    st->edges_traversed += e;
+    st->edges_examined += e;
+    st->host_bytes += o.edges[0] * rec;
+    st->topdown_host_bytes += o.edges[0] * rec;
+    st->hbm_bytes += hbm;  // no pass over the bitmap
+    st->topdown_hbm_bytes += hbm + 8 * bitmap_words(g.n) * o.levels;
+    const uint64_t host_parts = g.store.P - g.store.Pdev;
+    st->host_partitions_touched += (uint32_t)o.touched;
+    st->host_partitions_skipped += (uint32_t)(host_parts * o.levels - o.touched);
+    st->iterations += (uint32_t)o.levels;
+  }
+  return o;
+}
+
+// When k_small found a frontier too large after all, the general path runs
+// this many levels before the next try (doubled each time).
+struct SmallTry {
+  uint32_t wait = 0, step = 1;
+  bool ready() { return wait ? (wait--, false) : true; }
+  void done(const SmallOut &o) {
+    if (o.levels) {
+      step = 1;
+    } else {
+      wait = step;
+      step = step < 64 ? step * 2 : 64;
+    }
+  }
+};
+
 // Level-synchronous loop shared by BFS, CC and SSSP.  front[0] holds the
-// first frontier on entry.  Without events (w.ev null) no kernel time is
-// taken.
-static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st) {
+// first frontier on entry (from_src: {src}).  Small frontiers run in
+// k_small, many levels at once.  Without events (w.ev null) no kernel time
+// is taken.
+static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st, bool from_src,
+                       uint32_t src) {
   hipStream_t s = g.stream;
   const uint64_t words = g.n / 32 + 2;
   const bool timed = w.ev[0] && w.ev[1] && g.kernel_timing;
@@ -242,8 +353,19 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st) {
   int cur = 0;
   double expand_ms = 0;
   uint32_t launches = 0;
+  bool small = from_src;  // the frontier is known or likely to be small
+  SmallTry tries;
   const uint64_t t0 = now_ns();
   for (uint32_t L = 0;; L++) {
+    if (small) {
+      const SmallOut o = run_small(g, w, algo, w.front[cur].as<uint32_t>(), from_src, src, L + 2,
+                                   0xFFFFFFFFu, 0, timed, &expand_ms, st);
+      launches++;
+      from_src = false;
+      tries.done(o);
+      L += (uint32_t)o.levels;
+      if (o.state == 0) break;
+    }
     LevelCtr *c = d_ctr + (L & 1);
     // BFS: the level-L frontier holds the vertices at value L + 1
     launch_compact(g, w.qs, w.front[cur].as<uint32_t>(), c, s, 0,
@@ -267,6 +389,7 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st) {
     if (h.qn[0] + h.qn[1] == 0) break;
     stats_level(g, st, h);
     cur ^= 1;
+    small = small_frontier(h.qn[0] + h.qn[1], h.qw[0] + h.qw[1], algo) && tries.ready();
   }
   if (st) {
     st->ms = (now_ns() - t0) * 1e-6;
@@ -374,11 +497,15 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
   // one 170 us, a list probe level over 25K candidates 60 us.
   constexpr double TD_FIXED = 25e-6, TD_NS_TILE_ALL = 1.2, TD_NS_TILE = 9.7,
                    LIST_FIXED = 60e-6, LIST_NS_CAND = 0.03;
+  // A level k_small takes: its launches and round trip, and its edges on
+  // one CU.
+  constexpr double SMALL_FIXED = 25e-6, SMALL_NS_EDGE = 0.8;
   const double ntiles_d = (double)((g.n + TILE - 1) / TILE);
   uint64_t last_cand = 0;  // candidates the latest probe left
   // HBM side of a top-down level: tiles with frontier vertices taken as nf
   // vertices over the tiles at random
   auto td_hbm_cost = [&](uint64_t nf, uint64_t mf) {
+    if (small_frontier(nf, mf)) return SMALL_FIXED + (double)mf * SMALL_NS_EDGE * 1e-9;
     const double tiles_work = ntiles_d * -std::expm1(-(double)nf / ntiles_d);
     return TD_FIXED + ((double)nf * TD_NS_ENTRY + (double)mf * TD_NS_EDGE +
                        ntiles_d * TD_NS_TILE_ALL + tiles_work * TD_NS_TILE) * 1e-9;
@@ -548,6 +675,39 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
       }
     }
   };
+  // Levels k_small takes: no more edges than would make the rules below
+  // look at a bottom-up level (split store: host bytes / link rate against
+  // the probe; all edges in HBM: the edge ratio a caller has set, tested
+  // level by level -- the default ratio is for levels of the general path,
+  // where a top-down level costs as much as a bottom-up one).
+  const double ratio = host_share || !g.do_alpha_set ? 0.0 : g.do_alpha;
+  auto small_edges = [&](double probe_cost) {
+    const double e = host_share ? probe_cost * link / (double)rec : (double)SMALL_EDGES;
+    return (uint64_t)std::min(e, (double)SMALL_EDGES);
+  };
+  LevelCtr small_h;         // the frontier k_small left (in front[cur])
+  bool small_left = false;
+  // runs the levels from L on; true when the frontier ended empty, else
+  // (levels may be 0) small_h has its sums
+  uint64_t small_levels = 0;
+  auto small_run = [&](uint32_t L, bool from_src, uint64_t edge_max, uint64_t unvisited,
+                       const LevelSide *side) {
+    const SmallOut o = run_small(g, w, A_BFS, w.front[cur].as<uint32_t>(), from_src, src, L + 2,
+                                 0, 0, timed, &expand_ms, st, edge_max, ratio, unvisited, side);
+    launches++;
+    small_levels = o.levels;
+    visited_edges += o.edges[0] + o.edges[1];
+    if (o.levels) prev_nf = o.last_nf;
+    memset(&small_h, 0, sizeof small_h);
+    for (int q = 0; q < 2; q++) {
+      small_h.qn[q] = o.nf[q];
+      small_h.qw[q] = o.mf[q];
+    }
+    if (trace)
+      fprintf(stderr, "[thv] bfs L=%u %llu small levels, %llu vertices, %llu edges\n", L, o.levels,
+              o.vertices, o.edges[0] + o.edges[1]);
+    return o.state == 0;
+  };
   const uint64_t t0 = now_ns();
   for (uint32_t L = 0;; L++) {
     LevelCtr *c = d_ctr + (L & 1);
@@ -561,16 +721,19 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
     // and clears `dead` for the next level; a fused level has its probe or
     // compaction clear it.
     const bool fused = fused_next;
+    const bool resumed = small_left;  // the last levels ran in k_small
+    small_left = false;
     // Level 0 from a source whose whole list would not pay for a probe (or,
     // all edges in HBM, would not pass the edge-ratio rule) runs top-down
     // whatever its counts: its list expanded in one launch, no queue, no
     // readback.
     const uint64_t d0 = L == 0 ? g.h_off[src + 1] - g.h_off[src] : 0;
     const bool quick =
-        L == 0 && d0 > 0 &&
+        L == 0 && d0 > 0 && !resumed &&
         (host_share ? (double)d0 * rec / link + td_hbm_cost(1, d0) <=
                           (double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED
-                    : (double)d0 <= (double)(g.m - std::min<uint64_t>(g.m, d0)) / g.do_alpha);
+                    : (!g.do_alpha_set && d0 <= SMALL_EDGES) ||
+                          (double)d0 <= (double)(g.m - std::min<uint64_t>(g.m, d0)) / g.do_alpha);
     if (!quick && !fused) {
       LevelSide cs;
       cs.zero = dead;
@@ -581,6 +744,15 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
       cs.zctr = c_next;
       launch_compact(g, w.qs, front, c, s, CMP_COUNT_ONLY, w.val.as<uint32_t>(), L + 1, 1,
                      0xFFFFFFFFu, 0, nullptr, 0, nullptr, nullptr, &cs);
+    }
+    if (quick && d0 <= small_edges((double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED)) {
+      // one small list: this level and the small ones after it in one launch
+      if (small_run(L, true, small_edges((double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED),
+                    g.m, nullptr))
+        break;
+      fused_next = small_left = true;
+      L += (uint32_t)small_levels - 1;  // none: level 0 again, its sums known
+      continue;
     }
     if (quick) {
       // the frontier is {src}: its list expanded directly (the start cleared
@@ -599,13 +771,15 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
       cur = (cur + 1) % 3;
       continue;
     }
-    HIPC(hipStreamSynchronize(s));
-    finish_level(pend);
+    if (!resumed) {
+      HIPC(hipStreamSynchronize(s));
+      finish_level(pend);
+    }
     pend.valid = false;
-    const LevelCtr h = fused ? w.h_ctr[4] : w.h_ctr[L & 1];
+    const LevelCtr h = resumed ? small_h : fused ? w.h_ctr[4] : w.h_ctr[L & 1];
     uint32_t *clear = fused ? dead : nullptr;
     const uint64_t nf = h.qn[0] + h.qn[1], mf = h.qw[0] + h.qw[1];
-    if (fused && probed_last) last_cand = h.cand;
+    if (fused && probed_last && !resumed) last_cand = h.cand;
     if (nf == 0) break;
     visited_edges += mf;
     const uint64_t mu = g.m - std::min<uint64_t>(g.m, visited_edges);
@@ -663,7 +837,8 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
       }
     } else {
       // everything in HBM: the edge-ratio rule of Beamer et al.
-      if (!bu && (double)mf > (double)mu / g.do_alpha) bu = true;
+      if (!g.do_alpha_set && small_frontier(nf, mf)) bu = false;
+      else if (!bu && (double)mf > (double)mu / g.do_alpha) bu = true;
       else if (bu && (double)nf < (double)g.n / g.do_beta && nf < prev_nf) bu = false;
       // once a probe has left candidates, a bottom-up level costs a list
       // probe over them: taken when cheaper than the top-down compaction
@@ -672,6 +847,23 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
         bu_cost = list_cost();
         bu = bu_cost < td_cost;
       }
+    }
+    const uint64_t small_max =
+        small_edges(cand < 0 ? (double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED : list_cost());
+    if (!bu && !probed && !resumed && nf <= SPARSE_MAX && mf <= small_max) {
+      LevelSide zs;
+      zs.zero = clear;
+      zs.nzero = clear ? words : 0;
+      visited_edges -= mf;  // counted with its level
+      if (small_run(L, false, small_max, g.m - std::min<uint64_t>(g.m, visited_edges), &zs)) break;
+      if (small_levels) {
+        fused_next = small_left = true;
+        probed_last = false;
+        L += (uint32_t)small_levels - 1;
+        continue;
+      }
+      visited_edges += mf;
+      clear = nullptr;
     }
     prev_nf = nf;
     a.next = next;
@@ -787,7 +979,7 @@ void run_bfs(Graph &g, uint32_t src, uint32_t *out, thv_stats *st) {
                      dopt ? 6u : 0u);
   HIPC(hipGetLastError());
   if (dopt) bfs_direction_optimizing(g, src, st);
-  else value_loop(g, g.ws, A_BFS, st);
+  else value_loop(g, g.ws, A_BFS, st, true, src);
   finish_values(g, out, st, (uint32_t)(g.n + 1));
 }
 
@@ -806,7 +998,7 @@ void bfs_topdown_in(Graph &g, Workspace &w, uint32_t src, thv_stats *st) {
   hipLaunchKernelGGL(k_set_bit, dim3(1), dim3(1), 0, s, w.vis.as<uint32_t>(), src);
   hipLaunchKernelGGL(k_set_bit, dim3(1), dim3(1), 0, s, w.front[0].as<uint32_t>(), src);
   HIPC(hipStreamSynchronize(s));
-  value_loop(g, w, A_BFS, st);
+  value_loop(g, w, A_BFS, st, true, src);
 }
 
 void run_cc(Graph &g, uint32_t *out, thv_stats *st) {
@@ -833,7 +1025,7 @@ void run_cc(Graph &g, uint32_t *out, thv_stats *st) {
   hipLaunchKernelGGL(k_bits_prefix, dim3(fill_grid(words)), dim3(256), 0, s,
                      w.front[0].as<uint32_t>(), g.n, words);
   HIPC(hipStreamSynchronize(s));
-  value_loop(g, g.ws, A_CC, st);
+  value_loop(g, g.ws, A_CC, st, false, 0);
   finish_values(g, out, st, 0xFFFFFFFFu);
 }
 
@@ -846,7 +1038,7 @@ void run_cc(Graph &g, uint32_t *out, thv_stats *st) {
 // up by delta; the loop ends with the set empty.  The fixpoint is the
 // frontier Bellman-Ford one (shortest distances are unique); fewer edges
 // are relaxed twice because vertices wait for their bucket.
-static void sssp_delta(Graph &g, thv_stats *st) {
+static void sssp_delta(Graph &g, uint32_t src, thv_stats *st) {
   Workspace &w = g.ws;
   hipStream_t s = g.stream;
   ExpandArgs a = base_args(g);
@@ -858,8 +1050,20 @@ static void sssp_delta(Graph &g, thv_stats *st) {
   uint64_t thr = 1 + delta;  // values are 1 + distance
   double expand_ms = 0;
   uint32_t launches = 0;
+  bool from_src = true, small = true;  // the pending set is {src}
+  SmallTry tries;
   const uint64_t t0 = now_ns();
   for (uint32_t it = 0;; it++) {
+    if (small) {
+      const SmallOut o = run_small(g, w, A_SSSP, pend, from_src, src, 0,
+                                   (uint32_t)std::min<uint64_t>(thr, 0xFFFFFFFFull),
+                                   (uint32_t)delta, true, &expand_ms, st);
+      launches++;
+      from_src = false;
+      tries.done(o);
+      if (o.state == 0) break;
+      if (o.state == 1) thr = o.thr;
+    }
     LevelCtr *c = d_ctr + (it & 1);
     const uint32_t t32 = (uint32_t)std::min<uint64_t>(thr, 0xFFFFFFFFull);
     launch_compact(g, w.qs, pend, c, s, 0, nullptr, 0, 1, 0xFFFFFFFFu, 0, val, t32, pend);
@@ -878,6 +1082,7 @@ static void sssp_delta(Graph &g, thv_stats *st) {
       const uint32_t lo = reinterpret_cast<const uint32_t *>(w.h_aux + 3)[0];
       if (lo == 0xFFFFFFFFu) break;
       thr = (uint64_t)lo + delta;
+      small = false;
       continue;
     }
     a.ctr = c;
@@ -890,6 +1095,7 @@ static void sssp_delta(Graph &g, thv_stats *st) {
     expand_ms += ms;
     launches++;
     stats_level(g, st, h);
+    small = small_frontier(h.qn[0] + h.qn[1], h.qw[0] + h.qw[1], A_SSSP) && tries.ready();
   }
   if (st) {
     st->ms = (now_ns() - t0) * 1e-6;
@@ -911,8 +1117,8 @@ void run_sssp(Graph &g, uint32_t src, uint32_t *out, thv_stats *st) {
   HIPC(hipMemsetAsync(w.front[0].p, 0, words * 4, s));
   hipLaunchKernelGGL(k_set_bit, dim3(1), dim3(1), 0, s, w.front[0].as<uint32_t>(), src);
   HIPC(hipStreamSynchronize(s));
-  if (g.sssp_delta) sssp_delta(g, st);
-  else value_loop(g, g.ws, A_SSSP, st);
+  if (g.sssp_delta) sssp_delta(g, src, st);
+  else value_loop(g, g.ws, A_SSSP, st, true, src);
   finish_values(g, out, st, (uint32_t)(g.n + 1));
 }
 

@@ -1094,10 +1094,22 @@ void launch_fsum(Graph &g, const uint32_t *front, uint32_t *fsum, hipStream_t s)
   HIPC(hipGetLastError());
 }
 
+void launch_list_front(Graph &g, const uint32_t *front, uint32_t *list, uint32_t cap,
+                       unsigned int *count, hipStream_t s, const LevelSide *side) {
+  if (side && (side->pub || side->xpub || side->zctr))
+    fail(THV_ESTATE, "the frontier listing only clears words");
+  LevelSide zs;
+  if (side) zs = *side;
+  const uint64_t words = bitmap_words(g.n);
+  const uint32_t grid = (uint32_t)std::max<uint64_t>(
+      1, std::min<uint64_t>(div_up(words, 4 * CBS), 4ull * g.cus));
+  hipLaunchKernelGGL(k_list_front, dim3(grid), dim3(CBS), 0, s, front, words, list, cap, count,
+                     zs);
+  HIPC(hipGetLastError());
+}
+
 void launch_queue_sparse(Graph &g, QueueSet &w, const uint32_t *front, LevelCtr *ctr,
                          hipStream_t s, const LevelSide *side) {
-  if (side && (side->pub || side->xpub || side->zctr))
-    fail(THV_ESTATE, "the sparse queue only clears words");
   CompactArgs a;
   memset(&a, 0, sizeof a);
   a.rbit = g.store.d_rbit.as<uint32_t>();
@@ -1119,13 +1131,7 @@ void launch_queue_sparse(Graph &g, QueueSet &w, const uint32_t *front, LevelCtr 
   a.C = w.C;
   a.dmin = 1;
   a.dmax = 0xFFFFFFFFu;
-  LevelSide zs;
-  if (side) zs = *side;
-  const uint64_t words = bitmap_words(g.n);
-  const uint32_t grid = (uint32_t)std::max<uint64_t>(
-      1, std::min<uint64_t>(div_up(words, 4 * CBS), 4ull * g.cus));
-  hipLaunchKernelGGL(k_list_front, dim3(grid), dim3(CBS), 0, s, front, words,
-                     w.slist.as<uint32_t>(), SPARSE_MAX, &ctr->pad[0], zs);
+  launch_list_front(g, front, w.slist.as<uint32_t>(), SPARSE_MAX, &ctr->pad[0], s, side);
   hipLaunchKernelGGL(k_queue_list, dim3(1), dim3(QBS), 0, s, a, w.slist.as<const uint32_t>(),
                      SPARSE_MAX);
   HIPC(hipGetLastError());

@@ -467,7 +467,8 @@ void workspace_ensure(Graph &g) {
   for (auto &f : w.front) f.alloc(words * 4);
   w.vis.alloc(words * 4);
   w.fsum.alloc(fsum_words(g.n) * 4);
-  w.aux.alloc(16 * sizeof(unsigned long long));
+  w.aux.alloc(AUX_WORDS * sizeof(unsigned long long));
+  HIPC(hipMemset(w.aux.p, 0, AUX_WORDS * sizeof(unsigned long long)));
   w.val.alloc((g.n + 1) * 4);
   // fine-grained: a kernel's stores land in host memory without a cache
   // flush, and the host reads them after the stream sync
@@ -478,8 +479,8 @@ void workspace_ensure(Graph &g) {
     HIPC(hipHostGetDevicePointer((void **)&w.h_ctr_dev, w.h_ctr, 0));
   }
   if (!w.h_aux) {
-    HIPC(hipHostMalloc((void **)&w.h_aux, 16 * sizeof(unsigned long long), HF));
-    memset(w.h_aux, 0, 16 * sizeof(unsigned long long));
+    HIPC(hipHostMalloc((void **)&w.h_aux, AUX_WORDS * sizeof(unsigned long long), HF));
+    memset(w.h_aux, 0, AUX_WORDS * sizeof(unsigned long long));
     HIPC(hipHostGetDevicePointer((void **)&w.h_aux_dev, w.h_aux, 0));
   }
   for (auto &e : w.ev)

@@ -151,6 +151,7 @@ struct QueueSet {
   void ensure(const Graph &g, uint32_t C);
 };
 
+constexpr uint32_t AUX_WORDS = 32;
 struct Workspace {
   uint64_t n = 0, m = 0;
   QueueSet qs;
@@ -163,8 +164,8 @@ struct Workspace {
   DevMem fsum;                // frontier summary (launch_fsum)
   DevMem val;                 // u32 values (BFS / CC / SSSP)
   DevMem f0, f1, f2;          // PR arrays (fp32)
-  DevMem aux;                 // misc device counters (16 x u64)
-  // pinned, mapped readback (CTR_SLOTS LevelCtr, 16 u64): the host reads
+  DevMem aux;                 // misc device counters (AUX_WORDS x u64)
+  // pinned, mapped readback (CTR_SLOTS LevelCtr, AUX_WORDS u64): the host reads
   // them after a stream sync; kernels that finish a level write them
   // directly through the device addresses h_ctr_dev / h_aux_dev
   LevelCtr *h_ctr = nullptr;
@@ -208,6 +209,7 @@ struct Graph {
   bool sym = false;           // every edge has its reverse
   bool dir_opt = true;        // direction-optimising BFS when sym
   double do_alpha = 14.0, do_beta = 24.0;
+  bool do_alpha_set = false;  // the caller chose do_alpha: small frontiers heed it too
   // link cost model of a bottom-up level over a split store: each unvisited
   // vertex with host-resident edges costs one small zero-copy read
   double do_vertex_ns = 3.0;  // per long unvisited host list (measured on MI355X)
@@ -356,6 +358,54 @@ void launch_bu_probe(Graph &g, QueueSet &qs, const uint32_t *front, uint32_t *vi
                      const uint32_t *ccin = nullptr, uint32_t *cout = nullptr,
                      uint32_t *ccout = nullptr, const LevelSide *side = nullptr,
                      const uint32_t *fsum = nullptr);
+
+// Lists the vertices of a frontier bitmap: the first `cap` go to `list`, in
+// no order; *count (0 before) receives how many there are.  side (may be
+// null): words to clear.
+void launch_list_front(Graph &g, const uint32_t *front, uint32_t *list, uint32_t cap,
+                       unsigned int *count, hipStream_t s, const LevelSide *side = nullptr);
+
+// small.hip: levels with small frontiers, many per launch.
+// A level with more edges is left to the general path.  Measured on R-MAT
+// (edge factor 16, resident), ms a call: BFS scale 12, 16,384 edges 0.196,
+// 32,768 0.149, 131,072 0.153; scale 16 0.320 / 0.313 / 0.322.  SSSP edges
+// take an atomicMin and an 8-byte record: scale 14 0.51 / 0.51 / 0.47, scale
+// 16 1.12 / 1.13 / 1.21, scale 20 2.66 / 2.87 / 2.88.
+constexpr uint32_t SMALL_EDGES = 32768, SMALL_EDGES_SSSP = 16384;
+constexpr uint32_t SMALL_LEVELS = 4096;  // levels per launch (it then resumes from the bitmap)
+struct SmallOut {
+  unsigned long long state;     // 0 the frontier is empty, 1 the bitmap holds the rest,
+                                // 2 the listed frontier was too large (nothing done)
+  unsigned long long levels;    // levels run
+  unsigned long long thr;       // SSSP: the bucket bound reached
+  unsigned long long last_nf;   // vertices (with edges) of the last level run
+  unsigned long long nf[2], mf[2];  // state 1, BFS: the rest's vertices and edges (host, HBM)
+  unsigned long long vertices;  // vertices and edges (host, HBM) over the levels run
+  unsigned long long edges[2];
+  unsigned long long touched;   // host partitions touched, summed over the levels
+};
+struct SmallArgs {
+  const uint32_t *deg, *rbit, *vpart;
+  const uint8_t *pres;
+  const uint64_t *eptr;
+  uint32_t *ptouch;
+  uint32_t stamp;               // of the first level; each level takes the next one
+  bool split;                   // some lists are in host memory
+  uint32_t *val, *vis;          // vis: BFS only
+  uint32_t *front;              // bitmap of the frontier (SSSP: of the pending set)
+  const uint32_t *list;         // the frontier's vertices, *count of them; null: {src}
+  unsigned int *count;
+  uint32_t src;
+  uint32_t level_value;         // BFS: value of the vertices the first level finds
+  uint32_t thr, delta;          // SSSP: bucket bound and width
+  unsigned long long *far[2];   // SSSP: far lists, far_cap entries each
+  uint32_t far_cap;
+  uint32_t edge_max, max_levels;
+  double ratio;                 // BFS, > 0: a level also ends the run when its edges x ratio
+  uint64_t unvisited;           //   exceed the edges left (unvisited before the first level)
+  SmallOut *out;
+};
+void launch_small(Graph &g, Algo algo, const SmallArgs &a, hipStream_t s);
 
 struct BottomUpArgs {
   const uint32_t *llist, *loff;  // the probe's long lists, per wave region,

@@ -77,7 +77,7 @@ void lay_out(Graph &g, Workspace &w, Carver &c) {
   c.take(q.ptouch, ((uint64_t)g.store.P + 1) * 4);
   for (auto &f : w.front) c.take(f, words * 4);
   c.take(w.vis, words * 4);
-  c.take(w.aux, 16 * sizeof(unsigned long long));
+  c.take(w.aux, AUX_WORDS * sizeof(unsigned long long));
   c.take(w.val, (g.n + 1) * 4);
   q.n = g.n;
   q.m = g.m;
@@ -132,11 +132,12 @@ void run_bfs_noalloc(Graph &g, uint32_t src, uint32_t *out, thv_stats *st) {
     ~Unhook() { w.h_ctr = nullptr; }
   } unhook{w};
   hipStream_t s = g.stream;
-  // the array keeps the last call's contents: the segment sums and the
-  // partition stamps must start at zero (fill kernels, no memset nodes)
+  // the array keeps the last call's contents: the segment sums, the
+  // partition stamps and the counters must start at zero (fill kernels, no memset nodes)
   const uint64_t segs = (g.n / TILE + 1) / 64 + 1;
   launch_fill_u32(w.qs.ssum[0].as<uint32_t>(), 0u, segs * 4 * 2, s);
   launch_fill_u32(w.qs.ptouch.as<uint32_t>(), 0u, (uint64_t)g.store.P + 1, s);
+  launch_fill_u32(w.aux.as<uint32_t>(), 0u, AUX_WORDS * 2, s);
   bfs_topdown_in(g, w, src, st);
   if (out && g.n) {
     HIPC(hipMemcpyAsync(out, w.val.p, g.n * 4, hipMemcpyDeviceToHost, s));
