@@ -75,6 +75,27 @@ struct HostPinned {  // hipHostMalloc'd, mapped into the GPU address space
   void release();
 };
 
+// Large copies of device arrays to pageable host memory through a ring of
+// pinned slots (readback.cpp).  One call at a time per object.
+struct Readback {
+  // Below MIN_BYTES the ring's pinned allocation on a graph's first call
+  // (1.1 ms for 6 MB) outweighs what it saves (8 MB: 0.3 ms a call).  Slots
+  // of 4 MB copied 134 MB in 3.0 ms, of 2 MB in 3.5, of 1 MB in 4.4 (an event
+  // wait per slot); from 16 MB, where 2 MB slots are as fast (0.94 against
+  // 0.90 ms a BFS) and allocate half as much.
+  static constexpr size_t SLOTS = 3, SLOT = 2u << 20, SLOT_LARGE = 4u << 20, LARGE = 32u << 20,
+                          MIN_BYTES = 12u << 20, WORKERS = 8;
+  HostPinned ring;
+  hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr};
+  Readback() = default;
+  Readback(const Readback &) = delete;
+  Readback &operator=(const Readback &) = delete;
+  ~Readback();
+  void ensure(size_t slot);
+  // after what is queued on s; returns when out is filled
+  void copy(void *out, const void *dev, size_t bytes, hipStream_t s);
+};
+
 // ---- store -------------------------------------------------------------------
 
 struct Store {
@@ -173,6 +194,7 @@ struct Workspace {
   LevelCtr *h_ctr_dev = nullptr;
   unsigned long long *h_aux_dev = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // [2], [3]: probe
+  Readback rb;
   ~Workspace();
 };
 

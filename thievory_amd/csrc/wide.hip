@@ -395,7 +395,7 @@ void run_wide(Graph64 &g, int algo, uint64_t src, uint64_t *out, thv_stats *st,
     HIPC(hipStreamSynchronize(s));
   }
   if (digest3) memcpy(digest3, dg, sizeof dg);
-  if (out) HIPC(hipMemcpy(out, g.val.p, g.n * 8, hipMemcpyDeviceToHost));
+  if (out) g.rb.copy(out, g.val.p, g.n * 8, s);
   if (st) {
     st->ms = ms;
     st->iterations = (uint32_t)levels;

@@ -16,6 +16,7 @@ struct Graph64 {
   uint32_t P = 0, Pdev = 0;
   uint64_t dev_edges = 0, budget = UINT64_MAX;
   DevMem val, q[2], ctr, inq;    // values, queues, counters, queued marks
+  Readback rb;
   hipStream_t stream = nullptr;
   int device = 0, cus = 256;
   std::mutex mu;
