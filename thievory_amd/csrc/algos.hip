@@ -114,8 +114,8 @@ __device__ __forceinline__ void block_count_add(unsigned long long c, unsigned l
 // Push (pr_kernels.cu:846-860): residual above tol is applied and re-pushed.
 __global__ void __launch_bounds__(256)
 k_pr_push_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict__ deg,
-                 float *rank, float *delta, float *res, uint32_t *next,
-                 unsigned long long *aux) {
+                 float *rank, float *delta, float *res, const uint2 *__restrict__ hubtab,
+                 float *hubacc, uint32_t *next, unsigned long long *aux) {
   const uint64_t words64 = (n + 63) / 64;
   unsigned long long cnt = 0;
   for (uint64_t base = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) & ~63ull;
@@ -123,13 +123,23 @@ k_pr_push_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict_
     const uint64_t v = base + lane_id();
     bool act = false;
     if (v < n) {
-      const float r = res[v];
+      const uint2 t = hubtab[v >> 5];
+      const uint32_t bit = 1u << (v & 31);
+      const float r0 = res[v];
+      float r = r0;
+      if (t.x & bit) {  // a hub's records were summed apart
+        float *h = &hubacc[t.y + __popc(t.x & (bit - 1))];
+        r += *h;
+        *h = 0.0f;
+      }
       if (r > tol) {
         const uint32_t d = deg[v];
         rank[v] += r;
         delta[v] = d ? r * alpha / (float)d : 0.0f;
         res[v] = 0.0f;
         act = true;
+      } else if (r != r0) {
+        res[v] = r;  // waits for more
       }
     }
     const uint64_t b = __ballot(act);
@@ -1194,18 +1204,26 @@ void run_pr(Graph &g, int mode, float alpha, float tol, int max_iter, float *out
   HIPC(hipMemsetAsync(w.front[1].p, 0, words * 4, s));
   HIPC(hipStreamSynchronize(s));
 
-  ExpandArgs a = base_args(g);
-  a.pr_src = f1;  // push: delta, pull: contribution
-  a.pr_dst = f2;  // push: residual, pull: sum
-  if (mode == THV_PR_PUSH) {
+  PrArgs a;
+  memset(&a, 0, sizeof a);
+  for (int q = 0; q < 2; q++) {
+    a.qv[q] = w.qs.qv[q].as<uint32_t>();
+    a.qe[q] = w.qs.qe[q].as<unsigned long long>();
+    a.qc[q] = w.qs.qc[q].as<uint32_t>();
+  }
+  const bool push = mode == THV_PR_PUSH;
+  w.qs.C = push ? PR_CHUNK : 256u * (uint32_t)g.shape.ept;
+  a.eptr = g.store.d_eptr.as<uint64_t>();
+  a.src = f1;  // push: delta, pull: contribution
+  a.dst = f2;  // push: residual, pull: sum
+  if (push) {
     ensure_pr_hubs(g);
-    a.hubs = g.d_hubs.as<uint32_t>();
-    a.hubbit = g.d_hubbit.as<uint32_t>();
+    a.hubtab = g.d_hubtab.as<uint2>();
+    a.hubacc = g.d_hubacc.as<float>();
     a.nhubs = g.nhubs;
   }
   LevelCtr *d_ctr = w.qs.ctr.as<LevelCtr>();
   unsigned long long *aux = w.aux.as<unsigned long long>();
-  const Algo algo = mode == THV_PR_PUSH ? A_PR_PUSH : A_PR_PULL;
   int cur = 0;
   double expand_ms = 0;
   const uint64_t t0 = now_ns();
@@ -1215,12 +1233,12 @@ void run_pr(Graph &g, int mode, float alpha, float tol, int max_iter, float *out
     launch_compact(g, w.qs, w.front[cur].as<uint32_t>(), c, s);
     a.ctr = c;
     HIPC(hipEventRecord(w.ev[0], s));
-    launch_expand(g, algo, a, s);
+    launch_pr(g, push, a, s);
     HIPC(hipEventRecord(w.ev[1], s));
     HIPC(hipMemsetAsync(aux, 0, 8, s));
     if (mode == THV_PR_PUSH)
       hipLaunchKernelGGL(k_pr_push_update, dim3(ug), dim3(256), 0, s, n, alpha, tol,
-                         g.d_deg.as<uint32_t>(), rank, f1, f2,
+                         g.d_deg.as<uint32_t>(), rank, f1, f2, a.hubtab, a.hubacc,
                          w.front[cur ^ 1].as<uint32_t>(), aux);
     else
       hipLaunchKernelGGL(k_pr_pull_update, dim3(ug), dim3(256), 0, s, n, alpha, tol,

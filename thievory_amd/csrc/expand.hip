@@ -2,8 +2,8 @@
 //
 // Replaces the reference's warp-per-vertex edge kernels
 // (BFS32_Static/Demand/Filter_Kernel src/bfs/bfs_kernels.cu:4-76, 111-154,
-// 196-287; CC32_* src/cc/cc_kernels.cu; SSSP32_* src/sssp/sssp_kernels.cu;
-// PR32_* src/pr/pr_kernels.cu) with one kernel per algorithm that walks the
+// 196-287; CC32_* src/cc/cc_kernels.cu; SSSP32_* src/sssp/sssp_kernels.cu)
+// with one kernel per algorithm that walks the
 // level's work space -- the concatenated edge lists of the queued vertices --
 // in chunks of C = 256 * EPT edges (chunk.hpp), host-resident and HBM
 // chunks interleaved.
@@ -27,9 +27,6 @@
 //          (bfs_kernels.cu:29-44)
 //   CC   : atomicMin(val[w], val[v]) (cc_kernels.cu:50-66)
 //   SSSP : atomicMin(val[w], val[v] + weight) (sssp_kernels.cu:124-141)
-//   PR   : push atomicAdd(res[w], delta[v]) (pr_kernels.cu:539-542), into a
-//          per-block LDS sum first when w is one of the hub destinations;
-//          pull sum[v] += contrib[u] over in-edges (pr_kernels.cu:45-51)
 //   HINT  (store set-up, not a traversal): key64[v] = max over the edges
 //          of (deg[w] << 32 | ~w), reduced per entry in LDS
 //   CC link (union-find CC of a symmetric graph, cc.hip): link(v, w)
@@ -39,12 +36,6 @@
 namespace thv {
 
 constexpr int EBS = 256;
-
-// Slot of a hub id in the PR-push LDS table (Fibonacci hashing).
-__device__ __forceinline__ uint32_t hub_slot(uint32_t w) {
-  static_assert((PR_HUB_SLOTS & (PR_HUB_SLOTS - 1)) == 0, "power-of-two table");
-  return (w * 2654435761u) >> (32 - __builtin_ctz(PR_HUB_SLOTS));
-}
 
 // BFS relaxation of EPT edges whose destinations are loaded (an absent edge
 // is 0xFFFFFFFF), each phase issuing the memory operations of all EPT edges
@@ -100,36 +91,12 @@ __global__ void __launch_bounds__(EBS) k_expand(ExpandArgs a) {
   __shared__ uint32_t s_mask[NW];
   __shared__ uint32_t s_pre[NW];
   __shared__ unsigned long long s_base[C + 1];
-  // CC/SSSP: source value; PR pull, hint build, CC link: vertex id (PR push
-  // has no use for it).  PR push runs 2 blocks per CU, bound by LDS: a table
-  // of 1,024 hubs gave 3 blocks per CU but was slower (83 ms against 78 per
-  // expansion at R-MAT 26), the hub atomics weigh more than occupancy.
-  constexpr uint32_t US = ALGO == A_PR_PUSH ? 1 : C + 1;
-  __shared__ uint32_t s_u[US];
-  __shared__ float s_f[C + 1];     // PR push: delta; PR pull: partial sum
-  // PR push: per-block sums for the hub destinations (an open-addressing
-  // table of the hub ids, built at kernel start, flushed at the end)
-  constexpr uint32_t HS = ALGO == A_PR_PUSH ? PR_HUB_SLOTS : 1;
-  __shared__ uint32_t s_hk[HS];
-  __shared__ float s_hv[HS];
+  __shared__ uint32_t s_u[C + 1];  // CC/SSSP: source value; hint build, CC link: vertex id
 
   // A_BFS_NEXT: the discovered vertices' entries and edges per residency
   unsigned long long nfn[2] = {0, 0}, nfe[2] = {0, 0};
   const ChunkSrc cs = chunk_src(a.ctr, C);
   const uint32_t tid = threadIdx.x;
-  if (ALGO == A_PR_PUSH) {
-    for (uint32_t t = tid; t < HS; t += EBS) {
-      s_hk[t] = 0xFFFFFFFFu;
-      s_hv[t] = 0.0f;
-    }
-    __syncthreads();
-    for (uint32_t t = tid; t < a.nhubs; t += EBS) {
-      const uint32_t w = a.hubs[t];
-      uint32_t sl = hub_slot(w);
-      while (atomicCAS(&s_hk[sl], 0xFFFFFFFFu, w) != 0xFFFFFFFFu) sl = (sl + 1) & (HS - 1);
-    }
-    __syncthreads();
-  }
 
   for (uint32_t c = blockIdx.x; c < cs.total; c += gridDim.x) {
     int q;
@@ -149,11 +116,6 @@ __global__ void __launch_bounds__(EBS) k_expand(ExpandArgs a) {
         atomicOr(&s_mask[s >> 5], 1u << (s & 31));
         s_base[t] = a.eptr[v] - b * REC;
         if (ALGO == A_CC || ALGO == A_SSSP) s_u[t] = a.val[v];
-        if (ALGO == A_PR_PUSH) s_f[t] = a.pr_src[v];
-        if (ALGO == A_PR_PULL) {
-          s_u[t] = v;
-          s_f[t] = 0.0f;
-        }
         if (ALGO == A_HINT || ALGO == A_CC_LINK) s_u[t] = v;
       }
     }
@@ -220,32 +182,6 @@ __global__ void __launch_bounds__(EBS) k_expand(ExpandArgs a) {
         const uint32_t w = dst[j], bit = 1u << (w & 31);
         if (!(nw[j] & bit)) atomicOr(&a.next[w >> 5], bit);
       }
-    } else if (ALGO == A_PR_PUSH) {
-      // a hub destination adds into the block's LDS table (it is there:
-      // every hub was inserted), any other one atomically in HBM
-      uint32_t hb[EPT];
-#pragma unroll
-      for (int j = 0; j < EPT; j++) hb[j] = a.hubbit[dst[j] != 0xFFFFFFFFu ? dst[j] >> 5 : 0];
-#pragma unroll
-      for (int j = 0; j < EPT; j++) {
-        const uint32_t w = dst[j];
-        if (w == 0xFFFFFFFFu) continue;
-        const float d = s_f[ent[j]];
-        if ((hb[j] >> (w & 31)) & 1u) {
-          uint32_t sl = hub_slot(w);
-          while (s_hk[sl] != w) sl = (sl + 1) & (HS - 1);
-          atomicAdd(&s_hv[sl], d);
-        } else {
-          unsafeAtomicAdd(&a.pr_dst[w], d);
-        }
-      }
-    } else if (ALGO == A_PR_PULL) {  // dst[j] is an in-neighbour of the entry's vertex
-      float c[EPT];
-#pragma unroll
-      for (int j = 0; j < EPT; j++) c[j] = a.pr_src[dst[j] != 0xFFFFFFFFu ? dst[j] : 0];
-#pragma unroll
-      for (int j = 0; j < EPT; j++)
-        if (dst[j] != 0xFFFFFFFFu) atomicAdd(&s_f[ent[j]], c[j]);
     } else if (ALGO == A_CC_LINK) {
 #pragma unroll
       for (int j = 0; j < EPT; j++)
@@ -259,12 +195,6 @@ __global__ void __launch_bounds__(EBS) k_expand(ExpandArgs a) {
         if (dst[j] != 0xFFFFFFFFu)
           atomicMax(&s_base[ent[j]], ((unsigned long long)dw[j] << 32) | (0xFFFFFFFFu - dst[j]));
     }
-    if (ALGO == A_PR_PULL) {
-      __syncthreads();
-      for (uint32_t t = tid; t < ci.nent; t += EBS) {
-        if (chunk_rel(qe[ci.i0 + t], ci.e0) < C) unsafeAtomicAdd(&a.pr_dst[s_u[t]], s_f[t]);
-      }
-    }
     if (ALGO == A_HINT) {
       __syncthreads();
       for (uint32_t t = tid; t < ci.nent; t += EBS) {
@@ -273,11 +203,6 @@ __global__ void __launch_bounds__(EBS) k_expand(ExpandArgs a) {
       }
     }
     __syncthreads();
-  }
-  if (ALGO == A_PR_PUSH) {
-    __syncthreads();
-    for (uint32_t t = tid; t < HS; t += EBS)
-      if (s_hk[t] != 0xFFFFFFFFu && s_hv[t] != 0.0f) unsafeAtomicAdd(&a.pr_dst[s_hk[t]], s_hv[t]);
   }
   if (ALGO == A_BFS_NEXT) {  // one atomic per counter and block
     __shared__ unsigned long long s_n[EBS / 64];
@@ -393,12 +318,6 @@ void launch_expand(Graph &g, Algo a, const ExpandArgs &args, hipStream_t s) {
     case A_SSSP:
       if (!r8) fail(THV_ENOTSUP, "SSSP needs 8-byte {dst, weight} records");
       launch_t<A_SSSP, 8>(g, args, s);
-      break;
-    case A_PR_PUSH:
-      r8 ? launch_t<A_PR_PUSH, 8>(g, args, s) : launch_t<A_PR_PUSH, 4>(g, args, s);
-      break;
-    case A_PR_PULL:
-      r8 ? launch_t<A_PR_PULL, 8>(g, args, s) : launch_t<A_PR_PULL, 4>(g, args, s);
       break;
     case A_HINT:
       r8 ? launch_t<A_HINT, 8>(g, args, s) : launch_t<A_HINT, 4>(g, args, s);

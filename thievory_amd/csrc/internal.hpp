@@ -252,9 +252,10 @@ struct Graph {
   // 1 densest partitions first, 2 sparsest first with the short-list side area
   int store_layout = 0;
   // PageRank push: the destinations that receive the most records (from a
-  // 1-in-64 sample of the edge array), sorted, and their bitmap; blocks
-  // accumulate adds to them in LDS.  Built on the first push call.
-  DevMem d_hubs, d_hubbit;
+  // 1-in-16 sample of the edge array), summed in LDS (pr.hip): per 32
+  // vertices their hub bits and the index of the first, and the hubs' sums.
+  // Built on the first push call.
+  DevMem d_hubtab, d_hubacc;
   uint32_t nhubs = 0;
   bool hubs_built = false;
   ~Graph();
@@ -279,8 +280,7 @@ uint64_t now_ns();
 // (deg[w] << 32 | ~w).  A_CC_LINK: union-find link of every edge (val is
 // the parent array, err the step-guard flag).
 enum Algo {
-  A_BFS = 0, A_CC = 1, A_SSSP = 2, A_PR_PUSH = 3, A_PR_PULL = 4, A_BFS_NEXT = 5, A_HINT = 6,
-  A_CC_LINK = 7
+  A_BFS = 0, A_CC = 1, A_SSSP = 2, A_BFS_NEXT = 3, A_HINT = 4, A_CC_LINK = 5
 };
 
 struct ExpandArgs {
@@ -296,11 +296,6 @@ struct ExpandArgs {
   unsigned long long *key64;  // hint build: per-vertex best key
   uint32_t *err;            // CC link: step-guard flag
   uint32_t uf_steps;        // CC link: step guard
-  float *pr_src;            // PR push: delta; PR pull: contribution
-  float *pr_dst;            // PR push: residual; PR pull: sum
-  const uint32_t *hubs;     // PR push: hub ids (nhubs, sorted) and bitmap
-  const uint32_t *hubbit;
-  uint32_t nhubs;
   uint32_t level_value;     // BFS: value given to discovered vertices
   uint32_t C;
   int rec;
@@ -310,6 +305,25 @@ struct ExpandArgs {
   const uint32_t *rbit;
   LevelCtr *nctr;
 };
+
+// pr.hip: PageRank's edge kernels, over a compaction with chunks
+// (QueueSet::C) of PR_CHUNK edges for push, of the launch shape for pull.
+constexpr uint32_t PR_CHUNK = 512;
+constexpr uint32_t PR_HUBS = 32768;  // hub sums a block keeps in LDS (128 KB)
+struct PrArgs {
+  const uint32_t *qv[2];
+  const unsigned long long *qe[2];
+  const uint32_t *qc[2];
+  const LevelCtr *ctr;
+  const uint64_t *eptr;
+  const float *src;       // push: delta; pull: contribution
+  float *dst;             // push: residual; pull: sum (both added to)
+  const uint2 *hubtab;    // push: per 32 vertices, hub bits and the first one's index
+  float *hubacc;          // push: the hubs' sums (added to)
+  uint32_t nhubs;
+};
+void launch_pr(Graph &g, bool push, const PrArgs &a, hipStream_t s);
+void ensure_pr_hubs(Graph &g);
 
 // Level bookkeeping a launch does on the side, so a level needs no memset
 // or readback copy of its own (every field may be null / 0):
@@ -467,9 +481,6 @@ void launch_fsum(Graph &g, const uint32_t *front, uint32_t *fsum, hipStream_t s)
 void launch_expand(Graph &g, Algo a, const ExpandArgs &args, hipStream_t s);
 
 // algos.hip
-constexpr uint32_t PR_HUBS = 2048;       // hub table entries
-constexpr uint32_t PR_HUB_SLOTS = 4096;  // LDS hash slots (power of two)
-void ensure_pr_hubs(Graph &g);
 void run_bfs(Graph &g, uint32_t src, uint32_t *out, thv_stats *st);
 // Top-down BFS levels over a workspace the caller lays out (no allocation
 // here); w.h_ctr must point at 2 host LevelCtr, w.ev may be null.
