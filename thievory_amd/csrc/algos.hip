@@ -94,22 +94,10 @@ void launch_fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // PageRank update kernels.  One wave covers 64 consecutive vertices, so the
-// next-frontier words are written whole from a ballot (no atomics).  The
-// number of activated vertices is summed per block and added to aux[0] once
-// per block: an atomic per wave on that one address serialises (a million
-// of them took 10 ms per iteration at n = 2^26).
-
-// Adds each wave's count (held by lane 0) to *aux, one atomic per block.
-__device__ __forceinline__ void block_count_add(unsigned long long c, unsigned long long *aux) {
-  __shared__ unsigned long long s_c[256 / 64];
-  if (lane_id() == 0) s_c[threadIdx.x >> 6] = c;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (uint32_t w = 0; w < blockDim.x / 64; w++) t += s_c[w];
-    if (t) atomicAdd(aux, t);
-  }
-}
+// next-frontier words are written whole from a ballot (no atomics).  A block
+// that activated a vertex sets aux[0], with a plain store: an atomic per
+// block on one address serialises (51 us an update of 2M vertices, 10 with
+// the store).  Bound: HBM, 20-24 bytes a vertex.
 
 // Push (pr_kernels.cu:846-860): residual above tol is applied and re-pushed.
 __global__ void __launch_bounds__(256)
@@ -117,7 +105,7 @@ k_pr_push_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict_
                  float *rank, float *delta, float *res, const uint2 *__restrict__ hubtab,
                  float *hubacc, uint32_t *next, unsigned long long *aux) {
   const uint64_t words64 = (n + 63) / 64;
-  unsigned long long cnt = 0;
+  bool any = false;
   for (uint64_t base = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) & ~63ull;
        base < words64 * 64; base += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t v = base + lane_id();
@@ -146,10 +134,10 @@ k_pr_push_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict_
     if (lane_id() == 0) {
       next[base / 32] = (uint32_t)b;
       next[base / 32 + 1] = (uint32_t)(b >> 32);
-      cnt += __popcll(b);
     }
+    any |= b != 0;
   }
-  block_count_add(cnt, aux);
+  if (any && lane_id() == 0) *aux = 1ull;
 }
 
 // Pull (pr_kernels.cu:449-476): active vertices take their new sum and stay
@@ -159,7 +147,7 @@ k_pr_pull_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict_
                  const uint32_t *__restrict__ cur, float *rank, float *contrib, float *sum,
                  uint32_t *next, unsigned long long *aux) {
   const uint64_t words64 = (n + 63) / 64;
-  unsigned long long cnt = 0;
+  bool any = false;
   for (uint64_t base = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) & ~63ull;
        base < words64 * 64; base += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t v = base + lane_id();
@@ -177,10 +165,10 @@ k_pr_pull_update(uint64_t n, float alpha, float tol, const uint32_t *__restrict_
     if (lane_id() == 0) {
       next[base / 32] = (uint32_t)b;
       next[base / 32 + 1] = (uint32_t)(b >> 32);
-      cnt += __popcll(b);
     }
+    any |= b != 0;
   }
-  block_count_add(cnt, aux);
+  if (any && lane_id() == 0) *aux = 1ull;
 }
 
 __global__ void k_pr_push_init(uint64_t n, float alpha, const uint32_t *__restrict__ deg,
@@ -240,6 +228,7 @@ static ExpandArgs base_args(Graph &g, Workspace &w) {
 }
 static ExpandArgs base_args(Graph &g) { return base_args(g, g.ws); }
 
+constexpr int AUX_MIN = 3;     // aux / h_aux[3]: SSSP's smallest later pending value
 constexpr int AUX_COUNT = 14;  // aux[14]: the listed frontier's size (0 between launches)
 constexpr int AUX_SMALL = 16;  // aux / h_aux[16, 28): SmallOut
 static_assert(AUX_SMALL + sizeof(SmallOut) / 8 <= AUX_WORDS, "SmallOut fits the counters");
@@ -378,16 +367,28 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st, bool fr
     }
     LevelCtr *c = d_ctr + (L & 1);
     // BFS: the level-L frontier holds the vertices at value L + 1
+    // the count pass clears the next level's bitmap
+    LevelSide cs;
+    cs.zero = w.front[cur ^ 1].as<uint32_t>();
+    cs.nzero = words;
     launch_compact(g, w.qs, w.front[cur].as<uint32_t>(), c, s, 0,
-                   algo == A_BFS ? w.val.as<uint32_t>() : nullptr, L + 1);
-    HIPC(hipMemsetAsync(w.front[cur ^ 1].p, 0, words * 4, s));
+                   algo == A_BFS ? w.val.as<uint32_t>() : nullptr, L + 1, 1, 0xFFFFFFFFu, 0,
+                   nullptr, 0, nullptr, nullptr, &cs);
     a.ctr = c;
     a.next = w.front[cur ^ 1].as<uint32_t>();
     a.level_value = L + 2;
     if (timed) HIPC(hipEventRecord(w.ev[0], s));
     launch_expand(g, algo, a, s);
     if (timed) HIPC(hipEventRecord(w.ev[1], s));
-    HIPC(hipMemcpyAsync(&w.h_ctr[L & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, s));
+    if (w.h_ctr_dev) {
+      LevelSide ps;
+      ps.pub_src = c;
+      ps.pub = w.h_ctr_dev + (L & 1);
+      ps.npub = 1;
+      launch_publish(ps, s);
+    } else {
+      HIPC(hipMemcpyAsync(&w.h_ctr[L & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, s));
+    }
     HIPC(hipStreamSynchronize(s));
     const LevelCtr &h = w.h_ctr[L & 1];
     // every launch is counted, the last one (empty frontier, exits at once)
@@ -1098,6 +1099,11 @@ static void sssp_delta(Graph &g, uint32_t src, thv_stats *st) {
   uint64_t thr = 1 + delta;  // values are 1 + distance
   double expand_ms = 0;
   uint32_t launches = 0;
+  // the count pass of each round also finds the smallest pending value of
+  // the later buckets (~0 between rounds: the publishing launch resets it)
+  unsigned long long *aux = w.aux.as<unsigned long long>();
+  uint32_t *d_min = reinterpret_cast<uint32_t *>(aux + AUX_MIN);
+  launch_fill_u32(d_min, 0xFFFFFFFFu, 2, s);
   bool from_src = true, small = true;  // the pending set is {src}
   SmallTry tries;
   const uint64_t t0 = now_ns();
@@ -1114,30 +1120,31 @@ static void sssp_delta(Graph &g, uint32_t src, thv_stats *st) {
     }
     LevelCtr *c = d_ctr + (it & 1);
     const uint32_t t32 = (uint32_t)std::min<uint64_t>(thr, 0xFFFFFFFFull);
-    launch_compact(g, w.qs, pend, c, s, 0, nullptr, 0, 1, 0xFFFFFFFFu, 0, val, t32, pend);
-    HIPC(hipMemcpyAsync(&w.h_ctr[it & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, s));
+    launch_compact(g, w.qs, pend, c, s, 0, nullptr, 0, 1, 0xFFFFFFFFu, 0, val, t32, pend, d_min);
+    a.ctr = c;
+    HIPC(hipEventRecord(w.ev[0], s));
+    launch_expand(g, A_SSSP, a, s);
+    HIPC(hipEventRecord(w.ev[1], s));
+    LevelSide ps;
+    ps.pub_src = c;
+    ps.pub = w.h_ctr_dev + (it & 1);
+    ps.npub = 1;
+    ps.xsrc = ps.xset = aux + AUX_MIN;
+    ps.xval = ~0ull;
+    ps.xpub = w.h_aux_dev + AUX_MIN;
+    ps.nx = 1;
+    launch_publish(ps, s);
     HIPC(hipStreamSynchronize(s));
     const LevelCtr h = w.h_ctr[it & 1];
     if (h.qn[0] + h.qn[1] == 0) {
-      // bucket done: the smallest pending value opens the next one (none
-      // pending: done)
-      uint32_t *d_min = reinterpret_cast<uint32_t *>(w.aux.as<unsigned long long>() + 3);
-      launch_fill_u32(d_min, 0xFFFFFFFFu, 1, s);
-      launch_compact(g, w.qs, pend, c, s, CMP_COUNT_ONLY, nullptr, 0, 1, 0xFFFFFFFFu, 0, val,
-                     0xFFFFFFFFu, nullptr, d_min);
-      HIPC(hipMemcpyAsync(w.h_aux + 3, d_min, 4, hipMemcpyDeviceToHost, s));
-      HIPC(hipStreamSynchronize(s));
-      const uint32_t lo = reinterpret_cast<const uint32_t *>(w.h_aux + 3)[0];
+      // bucket done (the expansion had nothing to do): the smallest pending
+      // value opens the next one (none pending: done)
+      const uint32_t lo = (uint32_t)w.h_aux[AUX_MIN];
       if (lo == 0xFFFFFFFFu) break;
       thr = (uint64_t)lo + delta;
       small = false;
       continue;
     }
-    a.ctr = c;
-    HIPC(hipEventRecord(w.ev[0], s));
-    launch_expand(g, A_SSSP, a, s);
-    HIPC(hipEventRecord(w.ev[1], s));
-    HIPC(hipStreamSynchronize(s));
     float ms = 0;
     HIPC(hipEventElapsedTime(&ms, w.ev[0], w.ev[1]));
     expand_ms += ms;
@@ -1224,19 +1231,23 @@ void run_pr(Graph &g, int mode, float alpha, float tol, int max_iter, float *out
   }
   LevelCtr *d_ctr = w.qs.ctr.as<LevelCtr>();
   unsigned long long *aux = w.aux.as<unsigned long long>();
-  int cur = 0;
   double expand_ms = 0;
   const uint64_t t0 = now_ns();
   const int ug = (int)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, 4096));
-  for (int it = 0; it < max_iter; it++) {
-    LevelCtr *c = d_ctr + (it & 1);
+  // The host looks at an iteration's counters while the next one runs: one
+  // launched after the last (nothing active) reads and changes nothing.
+  // Iteration i's counters and events are slot i & 1's.
+  hipEvent_t *ev = w.ev;  // [0], [1] the expansion of slot 0, [2], [3] of slot 1
+  launch_fill_u32(reinterpret_cast<uint32_t *>(aux), 0u, 2, s);
+  auto launch = [&](int it) {
+    const int k = it & 1, cur = it & 1;
+    LevelCtr *c = d_ctr + k;
     launch_compact(g, w.qs, w.front[cur].as<uint32_t>(), c, s);
     a.ctr = c;
-    HIPC(hipEventRecord(w.ev[0], s));
+    HIPC(hipEventRecord(ev[2 * k], s));
     launch_pr(g, push, a, s);
-    HIPC(hipEventRecord(w.ev[1], s));
-    HIPC(hipMemsetAsync(aux, 0, 8, s));
-    if (mode == THV_PR_PUSH)
+    HIPC(hipEventRecord(ev[2 * k + 1], s));
+    if (push)
       hipLaunchKernelGGL(k_pr_push_update, dim3(ug), dim3(256), 0, s, n, alpha, tol,
                          g.d_deg.as<uint32_t>(), rank, f1, f2, a.hubtab, a.hubacc,
                          w.front[cur ^ 1].as<uint32_t>(), aux);
@@ -1245,25 +1256,36 @@ void run_pr(Graph &g, int mode, float alpha, float tol, int max_iter, float *out
                          g.d_outdeg.as<uint32_t>(), w.front[cur].as<uint32_t>(), rank, f1,
                          f2, w.front[cur ^ 1].as<uint32_t>(), aux);
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(&w.h_ctr[it & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, s));
-    HIPC(hipMemcpyAsync(w.h_aux, aux, 8, hipMemcpyDeviceToHost, s));
-    HIPC(hipStreamSynchronize(s));
-    float ms = 0;
-    HIPC(hipEventElapsedTime(&ms, w.ev[0], w.ev[1]));
-    expand_ms += ms;
-    const LevelCtr &h = w.h_ctr[it & 1];
+    LevelSide ps;  // the totals and whether a vertex is active, which is reset
+    ps.pub_src = c;
+    ps.pub = w.h_ctr_dev + k;
+    ps.npub = 1;
+    ps.xsrc = aux;
+    ps.xpub = w.h_aux_dev + k;
+    ps.nx = 1;
+    ps.xset = aux;
+    launch_publish(ps, s);
+    HIPC(hipEventRecord(w.done[k], s));
+  };
+  for (int it = 0; it < max_iter; it++) {
+    if (it == 0) launch(0);
+    if (it + 1 < max_iter) launch(it + 1);
+    const int k = it & 1;
+    HIPC(hipEventSynchronize(w.done[k]));
+    expand_ms += event_ms(ev[2 * k], ev[2 * k + 1]);
+    const LevelCtr &h = w.h_ctr[k];
     stats_level(g, st, h);
     if (st) {
       // push: 4-byte atomic read+write of the residual per edge in place of
       // the state read; pull: 4-byte contribution read per edge.
       const uint64_t e = h.qw[0] + h.qw[1];
-      st->hbm_bytes += (mode == THV_PR_PUSH ? 4 : 0) * e;
+      st->hbm_bytes += (push ? 4 : 0) * e;
       st->hbm_bytes += 20 * n;  // update pass over rank / delta / residual
+      st->expand_launches++;
     }
-    cur ^= 1;
-    if (st) st->expand_launches++;
-    if (w.h_aux[0] == 0) break;
+    if (w.h_aux[k] == 0) break;
   }
+  HIPC(hipStreamSynchronize(s));
   if (st) {
     st->ms = (now_ns() - t0) * 1e-6;
     st->expand_ms = expand_ms;

@@ -54,7 +54,7 @@ struct CompactArgs {
   uint32_t *ptouch;
   uint32_t stamp;
   LevelCtr *ctr;
-  uint32_t C;
+  uint32_t C, cshift;  // edges per chunk, a power of two
   uint32_t invert;     // select vertices whose bit is clear
   uint32_t no_chunks;  // skip the chunk-start table
   uint32_t *val;       // BFS: frontier vertices' level, written by k_tcount
@@ -63,7 +63,7 @@ struct CompactArgs {
   const uint32_t *fval;  // if set: only vertices with fval[v] < fthr
   uint32_t fthr;
   uint32_t *clear;       // if set (write pass): clear the selected vertices' bits here
-  uint32_t *minout;      // if set (count pass, with fval): atomicMin of the selected fval
+  uint32_t *minout;      // if set (count pass, with fval): atomicMin of the fval >= fthr
   LevelSide side;        // count pass: k_tcount clears, k_sscan publishes
 };
 
@@ -73,7 +73,7 @@ struct CompactArgs {
 // lane shuffle, then the degrees of all selected vertices of all rounds are
 // loaded together.  Round r of lane l is vertex base + 64 r + l.
 struct SubTile {
-  uint32_t fmin;       // smallest fval of a selected vertex (with fval), else ~0
+  uint32_t fmin;       // smallest fval >= fthr of a vertex otherwise selected, else ~0
   uint32_t act;        // bit r: vertex of round r is selected and its degree in range
   uint32_t dev;        // bit r: its edges are in HBM
   uint32_t raw;        // bit r: its frontier bit is set (before any inversion)
@@ -104,16 +104,20 @@ __device__ __forceinline__ void load_subtile(const CompactArgs &a, uint64_t base
 #pragma unroll
   for (uint32_t r = 0; r < ROUNDS; r++)
     t.d[r] = ((t.act >> r) & 1u) ? a.deg[base + r * 64 + lane] : 0u;
-  uint32_t fv[ROUNDS];
+  t.fmin = 0xFFFFFFFFu;
   if (a.fval) {
+    uint32_t fv[ROUNDS];
 #pragma unroll
     for (uint32_t r = 0; r < ROUNDS; r++) {
       fv[r] = 0xFFFFFFFFu;
       if ((t.act >> r) & 1u) fv[r] = a.fval[base + r * 64 + lane];
     }
 #pragma unroll
-    for (uint32_t r = 0; r < ROUNDS; r++)
-      if (fv[r] >= a.fthr) t.d[r] = 0;  // fails the value filter
+    for (uint32_t r = 0; r < ROUNDS; r++) {
+      if (fv[r] < a.fthr) continue;
+      if (t.d[r] >= a.dmin && t.d[r] <= a.dmax) t.fmin = min(t.fmin, fv[r]);
+      t.d[r] = 0;  // fails the value filter
+    }
   }
 #pragma unroll
   for (uint32_t r = 0; r < ROUNDS; r++) {
@@ -123,12 +127,6 @@ __device__ __forceinline__ void load_subtile(const CompactArgs &a, uint64_t base
     }
   }
   t.dev &= t.act;
-  t.fmin = 0xFFFFFFFFu;
-  if (a.fval) {
-#pragma unroll
-    for (uint32_t r = 0; r < ROUNDS; r++)
-      if ((t.act >> r) & 1u) t.fmin = min(t.fmin, fv[r]);
-  }
 }
 
 // Per-lane totals of a sub-tile: entries and edges per queue.
@@ -276,15 +274,35 @@ __device__ __forceinline__ void tile_bases(const CompactArgs &a, uint32_t tile, 
 // count pass gives it one vertex per round): the entries a lane writes are
 // consecutive, so one wave scan of the lanes' totals places them all, in
 // place of a scan per 64 vertices.  It selects exactly the vertices the
-// count pass counted.
+// count pass counted.  A lane's stores would be 64 bytes and more from its
+// neighbours', so the tile's entries are put in order in LDS first (edge
+// starts relative to the tile's, in 32 bits) and leave in whole lines; the
+// degrees come in four 16-byte loads.  Bound: HBM, 4 bytes read and 12
+// written per vertex; 4M vertices, all active, take 20 us (48 with a
+// store per entry and a 64-bit division per chunk start).
 constexpr uint32_t VPL = SUB / 64;
 static_assert(VPL == 16, "a lane's run is half a bitmap word");
 
+__device__ __forceinline__ void load_run(const uint32_t *p, uint32_t (&x)[VPL]) {
+  const uint4 *p4 = reinterpret_cast<const uint4 *>(p);
+#pragma unroll
+  for (uint32_t k = 0; k < VPL / 4; k++) {
+    const uint4 y = p4[k];
+    x[4 * k] = y.x;
+    x[4 * k + 1] = y.y;
+    x[4 * k + 2] = y.z;
+    x[4 * k + 3] = y.w;
+  }
+}
+
 __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
   __shared__ unsigned long long s[CBS / 64][4];
+  __shared__ uint32_t s_id[TILE], s_rel[TILE];  // host entries, then HBM ones
   const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   for (uint32_t tile = blockIdx.x; tile < a.ntiles; tile += gridDim.x) {
-    if (a.tcnt[2 * tile] == 0 && a.tcnt[2 * tile + 1] == 0) continue;
+    const uint32_t nh = a.tcnt[2 * tile], nd = a.tcnt[2 * tile + 1];
+    if (nh == 0 && nd == 0) continue;
+    const bool wide = (a.tdeg[2 * tile] | a.tdeg[2 * tile + 1]) >> 32;  // starts past 32 bits
     const uint64_t v0 = (uint64_t)tile * TILE + (uint64_t)wv * SUB + (uint64_t)lane * VPL;
     const uint32_t sh = (uint32_t)(v0 & 31);
     unsigned long long tb[4];
@@ -298,21 +316,25 @@ __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
     }
     uint32_t d[VPL];
 #pragma unroll
-    for (uint32_t r = 0; r < VPL; r++) d[r] = ((sel >> r) & 1u) ? a.deg[v0 + r] : 0u;
-    if (a.fval) {
-      uint32_t fv[VPL];
+    for (uint32_t r = 0; r < VPL; r++) d[r] = 0;
+    if (sel) {
+      load_run(a.deg + v0, d);  // padded to whole tiles
+      if (a.fval) {
+        uint32_t fv[VPL];
+        if (a.n - v0 >= VPL) {
+          load_run(a.fval + v0, fv);
+        } else {
 #pragma unroll
-      for (uint32_t r = 0; r < VPL; r++) {
-        fv[r] = 0;
-        if ((sel >> r) & 1u) fv[r] = a.fval[v0 + r];
+          for (uint32_t r = 0; r < VPL; r++) fv[r] = v0 + r < a.n ? a.fval[v0 + r] : 0u;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < VPL; r++)
+          if (fv[r] >= a.fthr) d[r] = 0;  // fails the value filter
       }
-#pragma unroll
-      for (uint32_t r = 0; r < VPL; r++)
-        if (fv[r] >= a.fthr) d[r] = 0;  // fails the value filter
     }
 #pragma unroll
     for (uint32_t r = 0; r < VPL; r++) {
-      if (d[r] < a.dmin || d[r] > a.dmax) {
+      if (!((sel >> r) & 1u) || d[r] < a.dmin || d[r] > a.dmax) {
         sel &= ~(1u << r);
         d[r] = 0;
       }
@@ -336,7 +358,9 @@ __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
       if ((dev >> r) & 1u) ed += d[r];
       else eh += d[r];
     }
-    const unsigned long long ich = wave_incl_scan(ch), icd = wave_incl_scan(cd);
+    // entries (at most TILE of each) scan as one word
+    const uint32_t ic = wave_incl_scan((uint32_t)(ch << 16 | cd));
+    const unsigned long long ich = ic >> 16, icd = ic & 0xFFFFu;
     const unsigned long long ieh = wave_incl_scan(eh), ied = wave_incl_scan(ed);
     if (lane == 63) {
       s[wv][0] = ich;
@@ -345,11 +369,12 @@ __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
       s[wv][3] = ied;
     }
     __syncthreads();
-    unsigned long long idx[2] = {tb[0] + ich - ch, tb[1] + icd - cd};
-    unsigned long long eb[2] = {tb[2] + ieh - eh, tb[3] + ied - ed};
+    // relative to the tile's bases
+    uint32_t idx[2] = {(uint32_t)(ich - ch), (uint32_t)(icd - cd)};
+    unsigned long long eb[2] = {ieh - eh, ied - ed};
     for (uint32_t w = 0; w < wv; w++) {
-      idx[0] += s[w][0];
-      idx[1] += s[w][1];
+      idx[0] += (uint32_t)s[w][0];
+      idx[1] += (uint32_t)s[w][1];
       eb[0] += s[w][2];
       eb[1] += s[w][3];
     }
@@ -361,14 +386,22 @@ __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
     for (uint32_t r = 0; r < VPL; r++) {
       if (!((sel >> r) & 1u)) continue;
       const int q = ((dev >> r) & 1u) ? Q_DEV : Q_HOST;
-      const unsigned long long i = idx[q]++, e0 = eb[q];
+      const uint32_t li = idx[q]++;
+      const unsigned long long le = eb[q], e0 = tb[2 + q] + le;
       eb[q] += d[r];
-      a.qv[q][i] = (uint32_t)(v0 + r);
-      a.qe[q][i] = e0;
+      const unsigned long long i = tb[q] + li;
+      if (wide) {
+        a.qv[q][i] = (uint32_t)(v0 + r);
+        a.qe[q][i] = e0;
+      } else {
+        const uint32_t at = q == Q_HOST ? li : nh + li;
+        s_id[at] = (uint32_t)(v0 + r);
+        s_rel[at] = (uint32_t)le;
+      }
       if (!a.no_chunks) {
         uint32_t *qc = a.qc[q];
-        for (unsigned long long c = (e0 + a.C - 1) / a.C; c * a.C < e0 + d[r]; c++)
-          qc[c] = (uint32_t)i;
+        const unsigned long long c1 = (e0 + d[r] + a.C - 1) >> a.cshift;
+        for (unsigned long long c = (e0 + a.C - 1) >> a.cshift; c < c1; c++) qc[c] = (uint32_t)i;
       }
       if (pf != pl) {
         const uint32_t p = a.vpart[v0 + r];
@@ -379,6 +412,17 @@ __global__ void __launch_bounds__(CBS, 4) k_twrite(CompactArgs a) {
       }
     }
     __syncthreads();
+    if (!wide) {
+      for (uint32_t t = threadIdx.x; t < nh; t += CBS) {
+        a.qv[Q_HOST][tb[0] + t] = s_id[t];
+        a.qe[Q_HOST][tb[0] + t] = tb[2] + s_rel[t];
+      }
+      for (uint32_t t = threadIdx.x; t < nd; t += CBS) {
+        a.qv[Q_DEV][tb[1] + t] = s_id[nh + t];
+        a.qe[Q_DEV][tb[1] + t] = tb[3] + s_rel[nh + t];
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -1043,8 +1087,8 @@ __global__ void __launch_bounds__(QBS) k_queue_list(CompactArgs a, const uint32_
     eb[q] += d;
     a.qv[q][k] = v;
     a.qe[q][k] = e0;
-    for (unsigned long long c = (e0 + a.C - 1) / a.C; c * a.C < e0 + d; c++)
-      a.qc[q][c] = (uint32_t)k;
+    const unsigned long long c1 = (e0 + d + a.C - 1) >> a.cshift;
+    for (unsigned long long c = (e0 + a.C - 1) >> a.cshift; c < c1; c++) a.qc[q][c] = (uint32_t)k;
     const uint32_t p = a.vpart[v];
     if (atomicExch(&a.ptouch[p], a.stamp) != a.stamp) th[a.pres[p] ? Q_DEV : Q_HOST]++;
   }
@@ -1085,6 +1129,11 @@ __global__ void __launch_bounds__(CBS) k_fsum(const uint32_t *front, uint64_t wo
 }
 
 }  // namespace
+
+static uint32_t chunk_shift(uint32_t C) {
+  if (!C || (C & (C - 1))) fail(THV_ESTATE, "chunks are a power of two of edges");
+  return (uint32_t)__builtin_ctz(C);
+}
 
 void launch_fsum(Graph &g, const uint32_t *front, uint32_t *fsum, hipStream_t s) {
   const uint64_t nbits = fsum_bits(g.n);
@@ -1129,6 +1178,7 @@ void launch_queue_sparse(Graph &g, QueueSet &w, const uint32_t *front, LevelCtr 
   }
   a.ctr = ctr;
   a.C = w.C;
+  a.cshift = chunk_shift(w.C);
   a.dmin = 1;
   a.dmax = 0xFFFFFFFFu;
   launch_list_front(g, front, w.slist.as<uint32_t>(), SPARSE_MAX, &ctr->pad[0], s, side);
@@ -1171,6 +1221,7 @@ void launch_compact(Graph &g, QueueSet &w, const uint32_t *front, LevelCtr *ctr,
   }
   a.ctr = ctr;
   a.C = w.C;
+  a.cshift = chunk_shift(w.C);
   a.invert = (mode & CMP_INVERT) ? 1u : 0u;
   a.no_chunks = (mode & CMP_NO_CHUNKS) ? 1u : 0u;
   a.val = (mode & (CMP_INVERT | CMP_WRITE_ONLY)) ? nullptr : val;

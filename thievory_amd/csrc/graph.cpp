@@ -90,6 +90,8 @@ Workspace::~Workspace() {
   if (h_aux) (void)hipHostFree(h_aux);
   for (auto &e : ev)
     if (e) (void)hipEventDestroy(e);
+  for (auto &e : done)
+    if (e) (void)hipEventDestroy(e);
 }
 
 Graph::~Graph() {
@@ -453,6 +455,8 @@ void workspace_ensure(Graph &g) {
     HIPC(hipHostGetDevicePointer((void **)&w.h_aux_dev, w.h_aux, 0));
   }
   for (auto &e : w.ev)
+    if (!e) HIPC(hipEventCreate(&e));
+  for (auto &e : w.done)
     if (!e) HIPC(hipEventCreate(&e));
   w.n = g.n;
   w.m = g.m;

@@ -194,6 +194,7 @@ struct Workspace {
   LevelCtr *h_ctr_dev = nullptr;
   unsigned long long *h_aux_dev = nullptr;
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // [2], [3]: probe
+  hipEvent_t done[2] = {nullptr, nullptr};  // PageRank: an iteration's counters are out
   Readback rb;
   ~Workspace();
 };
@@ -331,7 +332,7 @@ void ensure_pr_hubs(Graph &g);
 //     the launch reads or writes otherwise);
 //   pub_src -> pub: npub LevelCtr copied, once the launch's counters are
 //     final, to the host-mapped readback; xsrc -> xpub: nx u64 counters too;
-//   zctr: a LevelCtr reset to zero after that copy.
+//   zctr: a LevelCtr reset to zero after that copy; xset: a counter set.
 // The host reads the readback after a stream sync: the launch's completion
 // orders its stores to host memory before the sync returns.
 struct LevelSide {
@@ -344,6 +345,8 @@ struct LevelSide {
   unsigned long long *xpub = nullptr;
   uint32_t nx = 0;
   LevelCtr *zctr = nullptr;
+  unsigned long long *xset = nullptr;  // a u64 counter among xsrc set to xval
+  unsigned long long xval = 0;         //   after that copy
 };
 
 // Compaction modes: INVERT takes the vertices whose bit is CLEAR (the
@@ -356,7 +359,7 @@ enum { CMP_INVERT = 1, CMP_NO_CHUNKS = 2, CMP_COUNT_ONLY = 4, CMP_WRITE_ONLY = 8
 // fval / fthr: select only vertices with fval[v] < fthr.  clear: the write
 // pass clears the bits of the vertices it selects there (the front bitmap
 // itself, for a pending set).  minout (with fval): the count pass lowers
-// *minout to the smallest fval of a selected vertex.  side (count pass
+// *minout to the smallest fval >= fthr of a vertex that only fthr excludes.  side (count pass
 // only; ignored by WRITE_ONLY): the count kernel clears side->zero, the
 // scan publishes after writing the totals and resets side->zctr.
 void launch_compact(Graph &g, QueueSet &qs, const uint32_t *front, LevelCtr *ctr,

@@ -41,7 +41,10 @@ __device__ __forceinline__ void side_publish(const LevelSide &s, uint32_t lane,
     reinterpret_cast<unsigned long long *>(s.pub + slot)[k] = v;
     if (zin && c == s.zctr) *src = 0ull;
   }
-  if (s.xpub && lane < s.nx) s.xpub[lane] = s.xsrc[lane];
+  if (s.xpub && lane < s.nx) {
+    s.xpub[lane] = s.xsrc[lane];
+    if (s.xsrc + lane == s.xset) *s.xset = s.xval;
+  }
   if (s.zctr && !zin && lane < W) reinterpret_cast<unsigned long long *>(s.zctr)[lane] = 0ull;
   __threadfence_system();
 }
