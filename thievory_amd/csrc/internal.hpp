@@ -60,6 +60,11 @@ struct DevMem {
     own = false;
   }
   void release();
+  void swap(DevMem &o) {
+    std::swap(p, o.p);
+    std::swap(bytes, o.bytes);
+    std::swap(own, o.own);
+  }
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 

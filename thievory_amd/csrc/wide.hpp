@@ -8,14 +8,22 @@ namespace thv {
 
 struct Graph64 {
   uint64_t n = 0, k = 0, m = 0;  // vertices, listed vertices (with edges), edges
-  int rec = 8;                   // 8: u64 dst; 16: {u64 dst, u32 w, pad}
-  std::vector<uint64_t> h_ids, h_loff;
+  // numbered vertices: the listed ones, then the destinations without a list
+  uint64_t N = 0;
+  int rec = 8;                   // 8: u64 number; 16: {u64 number, u32 w, pad}
+  uint32_t seg_shift = 0;        // log2 of the records per list segment
+  std::vector<uint64_t> h_ids, h_loff, h_extra;
   HostPinned h_edges;            // every record, mapped
-  DevMem d_ids, d_loff, d_eptr;  // sorted listed ids, list offsets, list addresses
+  DevMem d_uid;                  // ids of the numbered vertices (both parts sorted)
+  DevMem d_loff, d_eptr;         // list offsets, list addresses (listed vertices)
   DevMem slab;                   // HBM-resident runs of lists
   uint32_t P = 0, Pdev = 0;
   uint64_t dev_edges = 0, budget = UINT64_MAX;
-  DevMem val, q[2], ctr, inq;    // values, queues, counters, queued marks
+  DevMem val, stamp, q[2], ctr;  // values, queue stamps, queues, counters
+  DevMem at;                     // gather buffer
+  unsigned long long *h_ctr = nullptr, *h_ctr_dev = nullptr;  // mapped readback
+  int last_algo = -1;            // whose values these are
+  uint64_t lone = ~0ull;         // its source, when that has no number
   Readback rb;
   hipStream_t stream = nullptr;
   int device = 0, cus = 256;
