@@ -419,6 +419,7 @@ int thv_device_info(char *name, size_t name_len, int *cus, uint64_t *hbm_bytes) 
 int thv_device_memory(uint64_t *free_bytes, uint64_t *total_bytes) {
   return guarded([&] {
     size_t f = 0, t = 0;
+    drop_idle_engines();  // memory that any call can have counts as free
     HIPC(hipMemGetInfo(&f, &t));
     if (free_bytes) *free_bytes = f;
     if (total_bytes) *total_bytes = t;

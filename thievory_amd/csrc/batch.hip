@@ -45,6 +45,12 @@ struct MsArgs {
   unsigned long long fmask;  // BFS: lanes this expansion pushes (others run bottom-up)
 };
 
+// *p |= x where that sets a bit (blocks that bring nothing new do not queue
+// for the address).
+__device__ __forceinline__ void or_new(unsigned long long *p, unsigned long long x) {
+  if (x & ~__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(p, x);
+}
+
 // BFS: lane per edge, lane masks staged per queue entry.
 template <int REC, int EPT>
 __global__ void __launch_bounds__(MBS) k_ms_bfs(MsArgs a) {
@@ -140,7 +146,7 @@ __global__ void __launch_bounds__(MBS) k_ms_bfs(MsArgs a) {
     atomicAdd(&a.acc[ACC_HASH + tid], s_hash[tid]);
     atomicAdd(&a.acc[ACC_CNT + tid], (unsigned long long)s_cnt[tid]);
   }
-  if (tid == 0 && s_lm) atomicOr(&a.acc[ACC_LM], s_lm);
+  if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
 }
 
 // ---- bottom-up BFS levels (symmetric graphs) ---------------------------------
@@ -233,7 +239,7 @@ __device__ __forceinline__ void bu_digest_flush(BuDigest &d, unsigned long long 
     atomicAdd(&acc[ACC_CNT + tid], (unsigned long long)s_cnt[tid]);
   }
   if (tid == 0) {
-    if (s_misc[0]) atomicOr(&acc[ACC_LM], s_misc[0]);
+    or_new(&acc[ACC_LM], s_misc[0]);
     if (s_misc[1]) atomicAdd(&acc[ACC_MU], s_misc[1]);
     if (s_misc[2]) atomicAdd(&acc[ACC_SCAN_HOST], s_misc[2]);
     if (s_misc[3]) atomicAdd(&acc[ACC_SCAN_HBM], s_misc[3]);
@@ -279,16 +285,25 @@ __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
   const uint32_t myval = a.level + 2 - a.voff[lane];
   BuDigest dg;
   const uint64_t nwaves = (uint64_t)gridDim.x * (MBS / 64);
-  for (uint64_t w0 = ((uint64_t)blockIdx.x * (MBS / 64) + (tid >> 6)) * 64; w0 < a.n;
-       w0 += nwaves * 64) {
-    const uint64_t w = w0 + lane;
-    uint32_t d = 0;
-    unsigned long long sw = 0, U = 0;
-    if (w < a.n) {
-      d = a.deg[w];
-      sw = a.seen[w];
+  const uint64_t wstart = ((uint64_t)blockIdx.x * (MBS / 64) + (tid >> 6)) * 64;
+  // the next step's degrees and seen masks load while this step's lists are
+  // scanned
+  uint32_t dn = 0;
+  unsigned long long sn = 0;
+  if (wstart + lane < a.n) {
+    dn = a.deg[wstart + lane];
+    sn = a.seen[wstart + lane];
+  }
+  for (uint64_t w0 = wstart; w0 < a.n; w0 += nwaves * 64) {
+    const uint64_t w = w0 + lane, wn = w + nwaves * 64;
+    const uint32_t d = dn;
+    const unsigned long long sw = sn;
+    unsigned long long U = 0;
+    if (wn < a.n) {
+      dn = a.deg[wn];
+      sn = a.seen[wn];
     }
-    if (d) U = a.act & ~sw;
+    if (w < a.n && d) U = a.act & ~sw;
     const bool lng = U && d > BU_SHORT;
     unsigned long long acc = 0;
     uint32_t scanned = 0;
@@ -438,10 +453,16 @@ __global__ void __launch_bounds__(MBS) k_ms_bu_long(MsBuArgs a) {
 // ranks it once; the wave then walks the 64 edges, broadcasting each with
 // readlane, with the source and destination distance rows of 8 edges in
 // flight before the first compare.
-constexpr uint32_t SSSP_C = 1024;  // edges per chunk (4 waves x 4 x 64)
+// Chunks of 1,024 edges (4 waves x 4 x 64), or of 256 where a level has too
+// few to fill the chip with those: a wave's edges are a serial chain (64 take
+// 20 us, 256 80).  Batches of 64 sources, ms a call with 1,024 / 256 only:
+// R-MAT 14 2.18 / 1.39, 20 8.24 / 7.96, 22 24.6 / 25.7; so 256 below 8 large
+// chunks per CU.
+constexpr uint32_t SSSP_C = 256, SSSP_LARGE = 1024;
 
+template <uint32_t C>
 __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
-  constexpr uint32_t C = SSSP_C, NW = C / 32;
+  constexpr uint32_t NW = C / 32;
   constexpr uint32_t WAVES = MBS / 64, PER_WAVE = C / WAVES;
   __shared__ uint32_t s_mask[NW], s_pre[NW];
   __shared__ unsigned long long s_base[C + 1];
@@ -457,7 +478,7 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
     int q;
     uint32_t cc;
     chunk_pick(cs, c, q, cc);
-    const ChunkInfo ci = chunk_info<C>(cs, a.qc, q, cc);
+    const ChunkInfo ci = chunk_info<C, C / SSSP_C>(cs, a.qc, q, cc);
     for (uint32_t t = tid; t < NW; t += MBS) s_mask[t] = 0;
     __syncthreads();
     for (uint32_t t = tid; t < ci.nent; t += MBS) {
@@ -560,7 +581,7 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
     __syncthreads();
   }
   __syncthreads();
-  if (tid == 0 && s_lm) atomicOr(&a.acc[ACC_LM], s_lm);
+  if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
 }
 
 struct AdmitArgs {
@@ -600,6 +621,42 @@ __global__ void __launch_bounds__(MBS) k_ms_lanebits(const unsigned long long *F
     const unsigned long long b = __ballot(v < n && (F[v] & lanes) != 0);
     if (lane < 2) bits[(w0 >> 5) + lane] = (uint32_t)(b >> (32 * lane));
   }
+}
+
+// A level's start in one launch: the buffers it writes (last used two levels
+// ago) and its counters cleared.  F holds a mask only where fb has a bit, so
+// the pass reads n / 8 bytes and writes those masks, not all n.
+__global__ void __launch_bounds__(MBS) k_ms_begin(unsigned long long *F, uint32_t *fb,
+                                                  uint64_t words, unsigned long long *acc) {
+  const uint32_t lane = threadIdx.x & 63;
+  if (blockIdx.x == 0 && threadIdx.x < 5)
+    acc[threadIdx.x < 1 ? ACC_LM : ACC_LONG + threadIdx.x - 1] = 0;
+  const uint64_t nw = (uint64_t)gridDim.x * (MBS / 64);
+  for (uint64_t w0 = ((uint64_t)blockIdx.x * (MBS / 64) + (threadIdx.x >> 6)) * 64; w0 < words;
+       w0 += nw * 64) {
+    const uint32_t x = w0 + lane < words ? fb[w0 + lane] : 0u;
+    if (x) fb[w0 + lane] = 0;
+    // two words (64 vertices) at a time, one vertex per lane
+    for (unsigned long long any = wave_ballot(x != 0); any;) {
+      const uint32_t i = (uint32_t)__builtin_ctzll(any) & ~1u;
+      any &= ~(3ull << i);
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)x, (int)i);
+      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)x, (int)i + 1);
+      if (((lane < 32 ? lo : hi) >> (lane & 31)) & 1u) F[(w0 + i) * 32 + lane] = 0;
+    }
+  }
+}
+
+// The level's results to the host: the lanes' counters and the compaction's.
+__global__ void __launch_bounds__(MBS) k_ms_publish(const unsigned long long *acc,
+                                                    unsigned long long *hacc,
+                                                    const LevelCtr *c, LevelCtr *hc) {
+  for (uint32_t i = threadIdx.x; i < ACC_WORDS; i += MBS) hacc[i] = acc[i];
+  constexpr uint32_t W = (uint32_t)(sizeof(LevelCtr) / 8);
+  if (c && threadIdx.x < W)
+    reinterpret_cast<unsigned long long *>(hc)[threadIdx.x] =
+        reinterpret_cast<const unsigned long long *>(c)[threadIdx.x];
+  __threadfence_system();
 }
 
 __global__ void k_ms_clear(unsigned long long *seen, uint64_t n, unsigned long long keep) {
@@ -693,8 +750,12 @@ MultiEngine::MultiEngine(Graph &gr, int al, uint32_t lanes, bool kf)
   }
   acc.alloc(ACC_WORDS * 8);
   HIPC(hipMemsetAsync(acc.p, 0, ACC_WORDS * 8, stream));
-  HIPC(hipHostMalloc((void **)&h_acc, ACC_WORDS * 8, hipHostMallocDefault));
-  HIPC(hipHostMalloc((void **)&h_ctr, 2 * sizeof(LevelCtr), hipHostMallocDefault));
+  // fine-grained and mapped: kernels write the counters there (Workspace)
+  constexpr unsigned HF = hipHostMallocMapped | hipHostMallocCoherent;
+  HIPC(hipHostMalloc((void **)&h_acc, ACC_WORDS * 8, HF));
+  HIPC(hipHostMalloc((void **)&h_ctr, 2 * sizeof(LevelCtr), HF));
+  HIPC(hipHostGetDevicePointer((void **)&h_acc_dev, h_acc, 0));
+  HIPC(hipHostGetDevicePointer((void **)&h_ctr_dev, h_ctr, 0));
   HIPC(hipStreamSynchronize(stream));
 }
 
@@ -710,12 +771,19 @@ MultiEngine::~MultiEngine() {
 uint64_t MultiEngine::bytes_needed(const Graph &g, int algo, uint32_t lanes, bool keep_full) {
   const uint64_t n = g.n, words = bitmap_words(n);
   uint64_t b = 2 * (words * 4 + (n + 1) * 8);                       // fb, F
-  b += 2 * ((n + 1) * 12) + 2 * (g.m / PR_CHUNK + 2) * 4;            // queues
+  b += 2 * ((n + 1) * 12) + 2 * (g.m / QC_MIN + 2) * 4;              // queues
   b += (n / TILE + 1) * TILE * 4;                                     // long-list queue
   if (algo == THV_ALGO_BFS)
     b += (n + 1) * 8 + words * 4 + (keep_full ? (uint64_t)lanes * n * 4 : 0);
   else b += (uint64_t)lanes * n * 4 + (keep_full ? n * 4 : 0);
   return b;
+}
+
+uint64_t MultiEngine::bytes() const {
+  uint64_t b = 0;
+  for (const DevMem *m : {&fb[0], &fb[1], &F[0], &F[1], &tbits, &seen, &dist, &full, &acc})
+    b += m->bytes;
+  return b + qs.bytes();
 }
 
 uint32_t MultiEngine::chunk() const {
@@ -751,7 +819,7 @@ void MultiEngine::launch_level() {
                        seen.as<unsigned long long>(), n, ~pend_clear);
     pend_clear = 0;
   }
-  if (pend_finish) {
+  if (pend_finish && (!finish_last || !active)) {
     HIPC(hipMemsetAsync(acc.as<unsigned long long>() + RES_HASH, 0, 192 * 8, stream));
     hipLaunchKernelGGL(k_ms_sssp_finish, dim3(grid_for(n, 2048)), dim3(MBS), 0, stream,
                        dist.as<uint32_t>(), n, L, pend_finish, (uint32_t)(n + 1), true,
@@ -784,17 +852,20 @@ void MultiEngine::launch_level() {
   }
   level_bu = false;
   if (active) {
-    HIPC(hipMemsetAsync(F[cur ^ 1].p, 0, (n + 1) * 8, stream));
-    HIPC(hipMemsetAsync(fb[cur ^ 1].p, 0, words * 4, stream));
-    HIPC(hipMemsetAsync(acc.as<unsigned long long>() + ACC_LM, 0, 8, stream));
+    hipLaunchKernelGGL(k_ms_begin, dim3(grid_for(words, 4 * g.cus)), dim3(MBS), 0, stream,
+                       F[cur ^ 1].as<unsigned long long>(), fb[cur ^ 1].as<uint32_t>(), words,
+                       acc.as<unsigned long long>());
     LevelCtr *c = qs.ctr.as<LevelCtr>() + (level & 1);
     if (algo == THV_ALGO_BFS && g.sym && g.dir_opt) {
       // direction: the frontier's edges against the edges of the vertices
       // some lane still misses (an upper bound kept since the last
       // bottom-up level; any admission resets it to m)
-      launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, CMP_COUNT_ONLY);
-      HIPC(hipMemcpyAsync(&h_ctr[level & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost,
-                          stream));
+      LevelSide cs;
+      cs.pub_src = c;
+      cs.pub = h_ctr_dev + (level & 1);
+      cs.npub = 1;
+      launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, CMP_COUNT_ONLY, nullptr, 0, 1,
+                     0xFFFFFFFFu, 0, nullptr, 0, nullptr, nullptr, &cs);
       HIPC(hipStreamSynchronize(stream));
       const uint64_t mf = h_ctr[level & 1].qw[0] + h_ctr[level & 1].qw[1];
       level_bu = BU_ALPHA * mf > mu_est && mf > n / 8;
@@ -825,12 +896,14 @@ void MultiEngine::launch_level() {
     }
     launched_expand = true;
   }
-  HIPC(hipMemcpyAsync(h_acc, acc.p, ACC_WORDS * 8, hipMemcpyDeviceToHost, stream));
+  const LevelCtr *c = qs.ctr.as<LevelCtr>() + (level & 1);
+  hipLaunchKernelGGL(k_ms_publish, dim3(1), dim3(MBS), 0, stream, acc.as<unsigned long long>(),
+                     h_acc_dev, launched_expand ? c : nullptr, h_ctr_dev + (level & 1));
+  HIPC(hipGetLastError());
 }
 
 void MultiEngine::launch_bottom_up(uint64_t lanes) {
   const uint64_t n = g.n;
-  HIPC(hipMemsetAsync(acc.as<unsigned long long>() + ACC_LONG, 0, 4 * 8, stream));
   MsBuArgs b;
   memset(&b, 0, sizeof b);
   b.eptr = g.store.d_eptr.as<uint64_t>();
@@ -912,16 +985,23 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
       // milliseconds, and short blocks let the work-groups of other streams
       // (a BFS cohort's levels) take CUs as they free up.  The chunk count
       // comes from the compaction just launched (one readback).
-      HIPC(hipMemcpyAsync(&h_ctr[level & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost,
-                          stream));
+      LevelSide ps;
+      ps.pub_src = c;
+      ps.pub = h_ctr_dev + (level & 1);
+      ps.npub = 1;
+      launch_publish(ps, stream);
       HIPC(hipStreamSynchronize(stream));
       const LevelCtr &h = h_ctr[level & 1];
-      const uint64_t chunks = (h.qw[0] + SSSP_C - 1) / SSSP_C + (h.qw[1] + SSSP_C - 1) / SSSP_C;
+      const bool large = h.qw[0] + h.qw[1] >= 8ull * g.cus * SSSP_LARGE;
+      const uint32_t C = large ? SSSP_LARGE : SSSP_C;
+      const uint64_t chunks = div_up(h.qw[0], C) + div_up(h.qw[1], C);
       const uint64_t sg = std::max<uint64_t>(1, std::min<uint64_t>(chunks, 1u << 30));
-      hipLaunchKernelGGL(k_ms_sssp, dim3((uint32_t)sg), dim3(MBS), 0, stream, a);
+      if (large)
+        hipLaunchKernelGGL(k_ms_sssp<SSSP_LARGE>, dim3((uint32_t)sg), dim3(MBS), 0, stream, a);
+      else
+        hipLaunchKernelGGL(k_ms_sssp<SSSP_C>, dim3((uint32_t)sg), dim3(MBS), 0, stream, a);
     }
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(&h_ctr[level & 1], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, stream));
   }
 }
 
@@ -1015,6 +1095,78 @@ void MultiEngine::copy_full(uint32_t q, uint32_t *out) {
   HIPC(hipStreamSynchronize(stream));
 }
 
+// Engines of finished batches, kept for the next batch on their graph: making
+// one (some 25 allocations, and as many frees) took 1.5-2.7 ms of a 64-source
+// batch, as long as its levels at R-MAT 22.  An engine that is running is
+// not here.  All of them together hold at most KEEP bytes; a graph's go when
+// it is closed or its store changes, and all when an allocation fails or the
+// free memory is asked for.
+class IdleEngines {
+ public:
+  static constexpr uint64_t KEEP = 4ull << 30;
+  static IdleEngines &get() {
+    static IdleEngines *p = new IdleEngines();  // never destroyed: HIP may be gone by then
+    return *p;
+  }
+  std::unique_ptr<MultiEngine> take(Graph &g, int algo, uint32_t k) {
+    std::unique_ptr<MultiEngine> e;
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      for (size_t i = 0; i < idle.size(); i++) {
+        MultiEngine &x = *idle[i];
+        if (&x.g != &g || x.algo != algo || (algo == THV_ALGO_BFS ? x.L < k : x.L != k)) continue;
+        e = std::move(idle[i]);
+        idle.erase(idle.begin() + i);
+        break;
+      }
+    }
+    if (e) e->qs.ensure(g, e->chunk());  // the launch shape may have changed
+    return e;
+  }
+  void put(std::unique_ptr<MultiEngine> e) {
+    const uint64_t b = e->bytes();
+    if (b > KEEP) return;
+    std::vector<std::unique_ptr<MultiEngine>> out;  // freed without the lock
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t i = 0; i < idle.size();) {
+      if (&idle[i]->g == &e->g && idle[i]->algo == e->algo) {
+        out.push_back(std::move(idle[i]));
+        idle.erase(idle.begin() + i);
+      } else {
+        i++;
+      }
+    }
+    uint64_t sum = b;
+    for (auto &x : idle) sum += x->bytes();
+    while (sum > KEEP && !idle.empty()) {  // the longest unused first
+      sum -= idle.front()->bytes();
+      out.push_back(std::move(idle.front()));
+      idle.erase(idle.begin());
+    }
+    idle.push_back(std::move(e));
+  }
+  // all engines, or those of one graph; how many there were
+  size_t drop(const Graph *g) {
+    std::vector<std::unique_ptr<MultiEngine>> out;
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t i = 0; i < idle.size();) {
+      if (!g || &idle[i]->g == g) {
+        out.push_back(std::move(idle[i]));
+        idle.erase(idle.begin() + i);
+      } else {
+        i++;
+      }
+    }
+    return out.size();
+  }
+
+ private:
+  std::mutex mu;
+  std::vector<std::unique_ptr<MultiEngine>> idle;
+};
+
+size_t drop_idle_engines(const Graph *g) { return IdleEngines::get().drop(g); }
+
 void run_batch(Graph &g, int algo, const uint32_t *srcs, uint32_t k, uint64_t *hash,
                uint64_t *reached, uint32_t *depth, uint32_t *full, thv_stats *st) {
   if (k == 0) {
@@ -1023,7 +1175,17 @@ void run_batch(Graph &g, int algo, const uint32_t *srcs, uint32_t k, uint64_t *h
   }
   for (uint32_t i = 0; i < k; i++)
     if (srcs[i] >= g.n) fail(THV_EINVAL, "source vertex out of range");
-  MultiEngine e(g, algo, k, full != nullptr);
+  // an engine kept from an earlier batch starts as a server's does between
+  // queries: its finished lanes are cleared when the new ones are admitted
+  std::unique_ptr<MultiEngine> own = full ? nullptr : IdleEngines::get().take(g, algo, k);
+  if (!own) {
+    // (a BFS engine's memory does not depend on its lanes: it serves any k)
+    const uint32_t lanes = algo == THV_ALGO_BFS && !full ? MultiEngine::MAXL : k;
+    own.reset(new MultiEngine(g, algo, lanes, full != nullptr));
+  }
+  MultiEngine &e = *own;
+  e.finish_last = true;
+  memset(&e.stats, 0, sizeof e.stats);
   for (uint32_t i = 0; i < k; i++) e.admit(srcs[i], i);
   std::vector<LaneResult> done;
   const uint64_t t0 = now_ns();
@@ -1044,6 +1206,7 @@ void run_batch(Graph &g, int algo, const uint32_t *srcs, uint32_t k, uint64_t *h
     if (reached) reached[r.tag] = r.reached;
     if (depth) depth[r.tag] = r.depth;
   }
+  if (!full) IdleEngines::get().put(std::move(own));
 }
 
 }  // namespace thv

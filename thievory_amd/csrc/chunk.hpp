@@ -51,14 +51,15 @@ struct ChunkInfo {
 
 // Entries [i0, i0 + nent) intersect the chunk; entry i0 contains its first
 // edge.  nent <= C + 1 because every queued vertex has at least one edge.
-template <uint32_t C>
+// (The table of chunk starts may be finer: one start per C / STEP edges.)
+template <uint32_t C, uint32_t STEP = 1>
 __device__ __forceinline__ ChunkInfo chunk_info(const ChunkSrc &s, const uint32_t *const *qc,
                                                int q, uint32_t cc) {
   ChunkInfo ci;
   ci.e0 = (unsigned long long)cc * C;
   ci.len = (uint32_t)min((unsigned long long)C, s.W[q] - ci.e0);
-  ci.i0 = qc[q][cc];
-  const uint32_t i1 = cc + 1 < s.nch[q] ? qc[q][cc + 1] : (uint32_t)(s.nq[q] - 1);
+  ci.i0 = qc[q][cc * STEP];
+  const uint32_t i1 = cc + 1 < s.nch[q] ? qc[q][(cc + 1) * STEP] : (uint32_t)(s.nq[q] - 1);
   ci.nent = i1 - ci.i0 + 1;
   return ci;
 }

@@ -43,6 +43,10 @@ void DevMem::alloc(size_t b) {
   release();
   if (b == 0) b = 8;
   hipError_t e = hipMalloc(&p, b);
+  if (e != hipSuccess && drop_idle_engines() > 0) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, b);
+  }
   if (e != hipSuccess) {
     p = nullptr;
     (void)hipGetLastError();
@@ -95,6 +99,7 @@ Workspace::~Workspace() {
 }
 
 Graph::~Graph() {
+  (void)drop_idle_engines(this);
   if (stream) {
     (void)hipStreamSynchronize(stream);
     (void)hipStreamDestroy(stream);
@@ -131,6 +136,7 @@ void graph_build_tables(Graph &g) {
 void store_ensure(Graph &g) {
   if (g.store.configured) return;
   size_t fr = 0, tot = 0;
+  drop_idle_engines();
   HIPC(hipMemGetInfo(&fr, &tot));
   const uint64_t reserve = g.n * 96 + (g.m / 256 + 1) * 16 + (256ull << 20);
   const uint64_t avail = fr > reserve ? (uint64_t)((fr - reserve) * 0.9) : 0;
@@ -192,6 +198,7 @@ void store_configure(Graph &g, uint64_t budget, uint32_t part_edges) {
   if (part_edges == 0) fail(THV_EINVAL, "partition_edges must be > 0");
   if (g.n >= 0xFFFFFFFFull) fail(THV_ENOTSUP, "graphs need fewer than 2^32-1 vertices");
   Store &s = g.store;
+  drop_idle_engines(&g);
   HIPC(hipStreamSynchronize(g.stream));
   s.configured = false;
   s.part_edges = part_edges;
@@ -387,6 +394,15 @@ void store_configure(Graph &g, uint64_t budget, uint32_t part_edges) {
   if (s.hint_reserved) build_parent_hints(g);
 }
 
+uint64_t QueueSet::bytes() const {
+  uint64_t b = ctr.bytes + ptouch.bytes + slist.bytes + scnt.bytes + llist.bytes + lcnt.bytes +
+               loff.bytes;
+  for (int k = 0; k < 2; k++)
+    b += qv[k].bytes + qe[k].bytes + qc[k].bytes + tcnt[k].bytes + tdeg[k].bytes +
+         ssum[k].bytes + sbase[k].bytes + clist[k].bytes + ccnt[k].bytes;
+  return b;
+}
+
 void QueueSet::ensure(const Graph &g, uint32_t chunk) {
   if (P != g.store.P || !ptouch.p) {
     ptouch.alloc((uint64_t)(g.store.P + 1) * 4);
@@ -416,13 +432,13 @@ void QueueSet::ensure(const Graph &g, uint32_t chunk) {
       sbase[k].alloc(segs * 4 * 8);
     }
   }
-  C = chunk;  // the table of chunk starts holds any chunk of PR_CHUNK edges or more
-  if (chunk < PR_CHUNK) fail(THV_ESTATE, "queue chunk below the table's");
+  C = chunk;  // the table of chunk starts holds any chunk of QC_MIN edges or more
+  if (chunk < QC_MIN) fail(THV_ESTATE, "queue chunk below the table's");
   if (n == g.n && m == g.m && ctr.p) return;
   for (int q = 0; q < 2; q++) {
     qv[q].alloc((g.n + 1) * 4);
     qe[q].alloc((g.n + 1) * 8);
-    qc[q].alloc((g.m / PR_CHUNK + 2) * 4);
+    qc[q].alloc((g.m / QC_MIN + 2) * 4);
   }
   ctr.alloc(CTR_SLOTS * sizeof(LevelCtr));
   n = g.n;

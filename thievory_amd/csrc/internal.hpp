@@ -155,6 +155,7 @@ struct Graph;
 // consumed by an expansion kernel.  Engines that run concurrently on
 // different streams own separate QueueSets.
 constexpr uint32_t TILE = 4096;  // vertices per compaction tile
+constexpr uint32_t QC_MIN = 256;  // fewest edges per chunk the table of chunk starts is sized for
 constexpr uint32_t PROBE_REGION = 1024;  // vertices per wave region of the bottom-up probe
 
 struct QueueSet {
@@ -175,6 +176,7 @@ struct QueueSet {
   DevMem loff;                //   with their regions' exclusive bases (+ total)
   DevMem clist[2], ccnt[2];   //   and candidates for the traversal's next probe
   void ensure(const Graph &g, uint32_t C);
+  uint64_t bytes() const;
 };
 
 constexpr uint32_t AUX_WORDS = 32;
@@ -211,7 +213,8 @@ struct Shape {
   int ept = 8;                // edges per thread per chunk (chunk = 256*ept)
   int probe_bpc = 8;          // bottom-up probe, short-list and early-exit
                               // grids = probe_bpc * CUs (persistent)
-  int batch_bpc = 8;          // multi-source bottom-up grids = batch_bpc * CUs
+  int batch_bpc = 4;          // multi-source bottom-up grids = batch_bpc * CUs (8: R-MAT 19
+                              // 1.63 against 1.43 ms a 64-source batch, 22 and 23 the same)
 };
 
 // ---- graph -------------------------------------------------------------------
@@ -510,6 +513,9 @@ Graph *rmat_generate(int scale, int edge_factor, double a, double b, double c,
                      bool transpose);
 
 // batch.hip
+// Frees the engines kept from finished batches (of one graph, or all);
+// returns how many there were.
+size_t drop_idle_engines(const Graph *g = nullptr);
 void run_batch(Graph &g, int algo, const uint32_t *srcs, uint32_t k,
                uint64_t *hash, uint64_t *reached, uint32_t *depth,
                uint32_t *full, thv_stats *st);

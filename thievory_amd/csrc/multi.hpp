@@ -43,8 +43,8 @@ struct MultiEngine {
   DevMem tbits;          // BFS: frontier vertices of the lanes a split level runs top-down
   DevMem seen, dist, full;
   DevMem acc;            // u64: hash[64] cnt[64] levelmask res_hash[64] res_cnt[64] res_depth[64]
-  unsigned long long *h_acc = nullptr;
-  LevelCtr *h_ctr = nullptr;
+  unsigned long long *h_acc = nullptr, *h_acc_dev = nullptr;  // mapped readback
+  LevelCtr *h_ctr = nullptr, *h_ctr_dev = nullptr;
   int cur = 0;
   uint32_t level = 0;
   thv_stats stats;
@@ -53,6 +53,8 @@ struct MultiEngine {
   uint64_t active = 0;         // lanes traversing
   uint64_t pend_finish = 0;    // SSSP lanes done, digest pending
   uint64_t pend_clear = 0;     // BFS lanes done, seen bits to clear before an admission
+  bool finish_last = false;    // digest the finished SSSP lanes in one pass, at the end
+                               // (a batch; a server wants each as soon as it is done)
   uint64_t finalizing = 0;     // lanes whose digest is in flight this level
   uint32_t voff[MAXL] = {};
   uint32_t last_val[MAXL] = {};
@@ -90,6 +92,7 @@ struct MultiEngine {
   MultiEngine &operator=(const MultiEngine &) = delete;
 
   static uint64_t bytes_needed(const Graph &g, int algo, uint32_t lanes, bool keep_full);
+  uint64_t bytes() const;                  // device memory held
   uint32_t chunk() const;                  // edges per expansion chunk
   uint64_t free_mask() const;
   uint32_t free_lanes() const { return (uint32_t)__builtin_popcountll(free_mask()); }

@@ -205,6 +205,7 @@ int thv_serve_start(thv_graph *gh, const thv_serve_cfg *cfg, thv_server **out) {
     uint64_t budget = cfg->scratch_bytes;
     if (budget == 0) {
       size_t fr = 0, tot = 0;
+      drop_idle_engines();
       HIPC(hipMemGetInfo(&fr, &tot));
       budget = fr / 2;
     }
