@@ -409,20 +409,22 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st, bool fr
   }
 }
 
-// Values other than `none`, added to *cnt: one pass at HBM rate (134 MB in
-// about 30 us; the host's pass over the copied array took 4 ms).
-__global__ void __launch_bounds__(256) k_count_ne(const uint32_t *val, uint64_t n, uint32_t none,
-                                                  unsigned long long *cnt) {
-  __shared__ unsigned long long sh[256 / 64];
-  const uint64_t t = blockIdx.x * 256ull + threadIdx.x, T = gridDim.x * 256ull;
+// Values other than `none`, added to *cnt.  Bound: HBM (134 MB in about 30 us;
+// the host's pass over the copied array took 4 ms).  One block per CU: each
+// ends with an atomic on one address (2,048 of them took 27 us whatever n).
+__global__ void __launch_bounds__(1024) k_count_ne(const uint32_t *val, uint64_t n, uint32_t none,
+                                                   unsigned long long *cnt) {
+  __shared__ unsigned long long sh[1024 / 64];
+  const uint64_t t = blockIdx.x * 1024ull + threadIdx.x, T = gridDim.x * 1024ull;
   const uint4 *v4 = reinterpret_cast<const uint4 *>(val);
   unsigned long long c = 0;
+#pragma unroll 4
   for (uint64_t i = t; i < n / 4; i += T) {
     const uint4 x = v4[i];
     c += (x.x != none) + (x.y != none) + (x.z != none) + (x.w != none);
   }
   for (uint64_t i = n / 4 * 4 + t; i < n; i += T) c += val[i] != none;
-  c = block_sum<256>(c, sh);
+  c = block_sum<1024>(c, sh);
   if (threadIdx.x == 0 && c) atomicAdd(cnt, c);
 }
 
@@ -431,24 +433,32 @@ constexpr int AUX_REACHED = 15;
 // shorter than two more launches and a copy.
 constexpr uint64_t COUNT_MIN = 1u << 17;
 
-// The values to the caller, and how many of them differ from `none`.
-static void finish_values(Graph &g, uint32_t *out, thv_stats *st, uint32_t none) {
+// The values to the caller, and how many of them differ from `none` (the
+// labels of CC all do).  The stream has drained.
+static void finish_values(Graph &g, uint32_t *out, thv_stats *st, uint32_t none,
+                          bool labels = false) {
   Workspace &w = g.ws;
   if (!out) return;
-  const bool dev = st && g.n >= COUNT_MIN;
+  const bool dev = st && !labels && g.n >= COUNT_MIN;
   if (dev) {
     uint32_t *c = reinterpret_cast<uint32_t *>(w.aux.as<unsigned long long>() + AUX_REACHED);
     launch_fill_u32(c, 0u, 2, g.stream);
-    hipLaunchKernelGGL(k_count_ne, dim3((uint32_t)std::min<uint64_t>(div_up(g.n, 1024),
-                                                                     8ull * g.cus)),
-                       dim3(256), 0, g.stream, w.val.as<uint32_t>(), g.n, none,
+    hipLaunchKernelGGL(k_count_ne, dim3((uint32_t)std::min<uint64_t>(div_up(g.n, 4096), g.cus)),
+                       dim3(1024), 0, g.stream, w.val.as<uint32_t>(), g.n, none,
                        reinterpret_cast<unsigned long long *>(c));
     HIPC(hipGetLastError());
-    HIPC(hipMemcpyAsync(w.h_aux + AUX_REACHED, c, 8, hipMemcpyDeviceToHost, g.stream));
+    LevelSide ps;
+    ps.xsrc = reinterpret_cast<unsigned long long *>(c);
+    ps.xpub = w.h_aux_dev + AUX_REACHED;
+    ps.nx = 1;
+    launch_publish(ps, g.stream);
   }
   w.rb.copy(out, w.val.p, g.n * 4, g.stream);
   if (!st) return;
-  if (dev) {
+  if (labels) {
+    st->reached = g.n;
+  } else if (dev) {
+    HIPC(hipStreamSynchronize(g.stream));
     st->reached = w.h_aux[AUX_REACHED];
   } else {
     uint64_t r = 0;
@@ -1056,26 +1066,21 @@ void run_cc(Graph &g, uint32_t *out, thv_stats *st) {
   hipStream_t s = g.stream;
   const uint64_t words = g.n / 32 + 2;
   stats_begin(st);
-  if (g.n) {
-    hipLaunchKernelGGL(k_iota_u32, dim3(fill_grid(g.n)), dim3(256), 0, s, w.val.as<uint32_t>(),
-                       g.n);
-  }
   if (g.sym && g.cc_union && g.n) {
-    HIPC(hipStreamSynchronize(s));
     if (cc_union_find(g, st)) {
-      finish_values(g, out, st, 0xFFFFFFFFu);
+      finish_values(g, out, st, 0xFFFFFFFFu, true);
       return;
     }
-    // a link hit its step guard: start over with label propagation
-    stats_begin(st);
+    stats_begin(st);  // a link hit its step guard: label propagation
+  }
+  if (g.n)
     hipLaunchKernelGGL(k_iota_u32, dim3(fill_grid(g.n)), dim3(256), 0, s, w.val.as<uint32_t>(),
                        g.n);
-  }
   hipLaunchKernelGGL(k_bits_prefix, dim3(fill_grid(words)), dim3(256), 0, s,
                      w.front[0].as<uint32_t>(), g.n, words);
   HIPC(hipStreamSynchronize(s));
   value_loop(g, g.ws, A_CC, st, false, 0);
-  finish_values(g, out, st, 0xFFFFFFFFu);
+  finish_values(g, out, st, 0xFFFFFFFFu, true);
 }
 
 // SSSP by delta-stepping (Meyer & Sanders 2003) over the same compaction and

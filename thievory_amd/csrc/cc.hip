@@ -6,14 +6,18 @@
 // graph its fixpoint labels every vertex with the smallest id of its
 // component.  Union-find with "larger root under smaller" hooking (uf.hpp)
 // ends with exactly those labels, and reads far fewer edges:
-//   1. link every vertex to its first two neighbours, compress (a vertex
-//      whose list is on the host links its parent hint instead, when the
-//      store holds hints: one HBM word, no request over the link);
+//   1. link every vertex to its first two neighbours, compress.  When the
+//      store holds parent hints, every vertex links its hint instead (its
+//      neighbour of largest degree: one HBM word, no list, and the trees
+//      meet at the hubs): the start makes a smaller hint the vertex's parent
+//      at once, a larger one is linked (R-MAT 23, edge factor 32, labels left
+//      in HBM: 0.53 ms with two records a vertex, 310 us of it this step;
+//      0.25 with the hints);
 //   2. sample 1024 vertices: the most frequent root is the giant component;
 //   3. link the remaining lists of the vertices outside it (its own
 //      members need nothing more: an edge to a non-member is linked from
-//      the other side, which the graph's symmetry guarantees; a hinted
-//      host list counts as remaining whatever its length), compress.
+//      the other side, which the graph's symmetry guarantees; with hints a
+//      list has one linked record, not two), compress.
 // Directed graphs keep label propagation (the labels there are not
 // components).
 #include <algorithm>
@@ -30,23 +34,46 @@ namespace {
 constexpr int UBS = 256;
 constexpr uint32_t CC_SAMPLES = 1024;
 
-// Step 1, one vertex per thread: its first two records, then the links;
-// with hints (nullable), a host list's vertex links its hint instead.
+// The start: every vertex its own parent, or (hint given) its parent hint
+// where that is a smaller id -- parents point to smaller ids, so the trees
+// are sound without a link.  cnt[1]: hints taken; cnt[0..2] start at zero.
+__global__ void __launch_bounds__(UBS) k_cc_start(uint32_t *comp, const uint32_t *hint,
+                                                  uint64_t n) {
+  for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v < n;
+       v += (uint64_t)gridDim.x * UBS) {
+    const uint32_t h = hint ? hint[v] : NO_HINT;  // NO_HINT is past every id
+    comp[v] = h < v ? h : (uint32_t)v;
+  }
+}
+
+// Step 1 with hints: the larger ones are linked.
+__global__ void __launch_bounds__(UBS) k_cc_hint(const uint32_t *hint, uint64_t n, uint32_t *comp,
+                                                 uint32_t *err, uint32_t steps,
+                                                 unsigned long long *cnt) {
+  __shared__ unsigned long long sh[UBS / 64];
+  unsigned long long taken = 0;
+  for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v < n;
+       v += (uint64_t)gridDim.x * UBS) {
+    const uint32_t h = hint[v];
+    taken += h != NO_HINT;
+    if (h != NO_HINT && h > v) uf_link((uint32_t)v, h, comp, err, steps);
+  }
+  taken = block_sum<UBS>(taken, sh);
+  if (threadIdx.x == 0 && taken) atomicAdd(&cnt[1], taken);
+}
+
+// Step 1 without hints, one vertex per thread: its first two records, then
+// the links.
 template <int REC>
 __global__ void __launch_bounds__(UBS)
-k_cc_first(const uint64_t *eptr, const uint32_t *deg, const uint32_t *rbit, const uint32_t *hint,
-           uint64_t n, uint32_t *comp, uint32_t *err, uint32_t steps, unsigned long long *cnt) {
+k_cc_first(const uint64_t *eptr, const uint32_t *deg, const uint32_t *rbit, uint64_t n,
+           uint32_t *comp, uint32_t *err, uint32_t steps, unsigned long long *cnt) {
   __shared__ unsigned long long sh[UBS / 64];
-  unsigned long long rd[2] = {0, 0};  // records read (host, HBM); a hint counts as HBM
+  unsigned long long rd[2] = {0, 0};  // records read (host, HBM)
   for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v < n;
        v += (uint64_t)gridDim.x * UBS) {
     const uint32_t d = deg[v];
     if (!d) continue;
-    if (hint && !((rbit[v >> 5] >> (v & 31)) & 1u)) {
-      uf_link((uint32_t)v, hint[v], comp, err, steps);  // d > 0: a neighbour
-      rd[1] += 1;
-      continue;
-    }
     const unsigned long long b = eptr[v];
     const uint32_t w0 = *reinterpret_cast<const uint32_t *>(b);
     const uint32_t w1 = d > 1 ? *reinterpret_cast<const uint32_t *>(b + REC) : w0;
@@ -75,25 +102,17 @@ __global__ void k_cc_sample(const uint32_t *comp, uint64_t n, uint32_t *out) {
 }
 
 // Vertices whose remaining lists are linked in step 3: a root other than
-// the giant's, and more than two records or (hinted) a host list.  One lane
+// the giant's, and more records than step 1 linked (`linked`).  One lane
 // per vertex; lanes 0 and 32 write the wave's two bitmap words.
 __global__ void __launch_bounds__(UBS)
-k_cc_rest(const uint32_t *comp, const uint32_t *deg, const uint32_t *rbit, bool hinted,
-          uint64_t n, uint32_t giant, uint32_t *bits) {
+k_cc_rest(const uint32_t *comp, const uint32_t *deg, uint32_t linked, uint64_t n, uint32_t giant,
+          uint32_t *bits, uint64_t words) {
   const uint32_t lane = threadIdx.x & 63;
-  for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v - lane < n;
+  for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v - lane < words * 32;
        v += (uint64_t)gridDim.x * UBS) {
-    bool sel = false;
-    if (v < n) {
-      const uint32_t d = deg[v];
-      const bool rest = d > 2 || (hinted && d > 0 && !((rbit[v >> 5] >> (v & 31)) & 1u));
-      sel = rest && comp[v] != giant;
-    }
+    const bool sel = v < n && deg[v] > linked && comp[v] != giant;
     const unsigned long long b = __ballot(sel);
-    if (lane == 0 || lane == 32) {
-      const uint64_t w = v >> 5;
-      if (w < (n + 31) / 32) bits[w] = (uint32_t)(b >> lane);
-    }
+    if ((lane == 0 || lane == 32) && v >> 5 < words) bits[v >> 5] = (uint32_t)(b >> lane);
   }
 }
 
@@ -110,19 +129,23 @@ bool cc_union_find(Graph &g, thv_stats *st) {
   uint32_t *comp = w.val.as<uint32_t>();
   unsigned long long *aux = w.aux.as<unsigned long long>();
   uint32_t *err = reinterpret_cast<uint32_t *>(aux + 2);
-  HIPC(hipMemsetAsync(aux, 0, 3 * 8, s));  // [0], [1] records read, [2] error flag
+  launch_fill_u32(reinterpret_cast<uint32_t *>(aux), 0u, 6, s);  // [0], [1] records, [2] error
   const uint64_t t0 = now_ns();
   const int grid = grid_for(n, 16 * g.cus);
   const uint32_t steps = g.uf_max_steps;
   const uint64_t *eptr = g.store.d_eptr.as<uint64_t>();
   const uint32_t *deg = g.d_deg.as<uint32_t>(), *rbit = g.store.d_rbit.as<uint32_t>();
   const uint32_t *hint = g.store.d_hint.as<uint32_t>();  // null without hints
-  if (g.rec == 8)
-    hipLaunchKernelGGL(k_cc_first<8>, dim3(grid), dim3(UBS), 0, s, eptr, deg, rbit, hint, n, comp,
-                       err, steps, aux);
+  hipLaunchKernelGGL(k_cc_start, dim3(grid), dim3(UBS), 0, s, comp, hint, n);
+  const int lgrid = grid_for(n, 4 * g.cus);  // ends with an atomic per block
+  if (hint)
+    hipLaunchKernelGGL(k_cc_hint, dim3(lgrid), dim3(UBS), 0, s, hint, n, comp, err, steps, aux);
+  else if (g.rec == 8)
+    hipLaunchKernelGGL(k_cc_first<8>, dim3(grid), dim3(UBS), 0, s, eptr, deg, rbit, n, comp, err,
+                       steps, aux);
   else
-    hipLaunchKernelGGL(k_cc_first<4>, dim3(grid), dim3(UBS), 0, s, eptr, deg, rbit, hint, n, comp,
-                       err, steps, aux);
+    hipLaunchKernelGGL(k_cc_first<4>, dim3(grid), dim3(UBS), 0, s, eptr, deg, rbit, n, comp, err,
+                       steps, aux);
   hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(UBS), 0, s, comp, n, err, steps);
   // the sample lands in the probe's short-list buffer (unused here; at
   // least one tile = 16 KB, CC_SAMPLES x 4 = 4 KB), then on the host
@@ -142,9 +165,8 @@ bool cc_union_find(Graph &g, thv_stats *st) {
     }
   // step 3: the rest of the lists outside the giant component
   uint32_t *bits = w.front[0].as<uint32_t>();
-  HIPC(hipMemsetAsync(bits, 0, words * 4, s));
-  hipLaunchKernelGGL(k_cc_rest, dim3(grid), dim3(UBS), 0, s, comp, deg, rbit, hint != nullptr, n,
-                     giant, bits);
+  hipLaunchKernelGGL(k_cc_rest, dim3(grid), dim3(UBS), 0, s, comp, deg, hint ? 1u : 2u, n, giant,
+                     bits, words);
   LevelCtr *c = w.qs.ctr.as<LevelCtr>();
   launch_compact(g, w.qs, bits, c, s);
   ExpandArgs a = expand_args(g, w.qs);
@@ -156,8 +178,14 @@ bool cc_union_find(Graph &g, thv_stats *st) {
   launch_expand(g, A_CC_LINK, a, s);
   HIPC(hipEventRecord(w.ev[1], s));
   hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(UBS), 0, s, comp, n, err, steps);
-  HIPC(hipMemcpyAsync(w.h_aux, aux, 3 * 8, hipMemcpyDeviceToHost, s));
-  HIPC(hipMemcpyAsync(&w.h_ctr[0], c, sizeof(LevelCtr), hipMemcpyDeviceToHost, s));
+  LevelSide ps;
+  ps.pub_src = c;
+  ps.pub = w.h_ctr_dev;
+  ps.npub = 1;
+  ps.xsrc = aux;
+  ps.xpub = w.h_aux_dev;
+  ps.nx = 3;
+  launch_publish(ps, s);
   HIPC(hipStreamSynchronize(s));
   if (w.h_aux[2]) return false;  // a link hit its step guard: not trusted
   if (st) {

@@ -81,23 +81,21 @@ struct HostPinned {  // hipHostMalloc'd, mapped into the GPU address space
 };
 
 // Large copies of device arrays to pageable host memory through a ring of
-// pinned slots (readback.cpp).  One call at a time per object.
+// pinned slots (readback.cpp).
 struct Readback {
-  // Below MIN_BYTES the ring's pinned allocation on a graph's first call
-  // (1.1 ms for 6 MB) outweighs what it saves (8 MB: 0.3 ms a call).  Slots
-  // of 4 MB copied 134 MB in 3.0 ms, of 2 MB in 3.5, of 1 MB in 4.4 (an event
-  // wait per slot); from 16 MB, where 2 MB slots are as fast (0.94 against
-  // 0.90 ms a BFS) and allocate half as much.
-  static constexpr size_t SLOTS = 3, SLOT = 2u << 20, SLOT_LARGE = 4u << 20, LARGE = 32u << 20,
-                          MIN_BYTES = 12u << 20, WORKERS = 8;
-  HostPinned ring;
-  hipEvent_t ev[SLOTS] = {nullptr, nullptr, nullptr};
-  Readback() = default;
+  // Slots of 4 MB copied 134 MB in 3.0 ms, of 2 MB in 3.5, of 1 MB in 4.4 (an
+  // event wait per slot); smaller arrays take smaller slots, which are as fast
+  // there and allocate less on the process's first copy (6 MB: 1.1 ms).  An 8
+  // MB array gains 0.2 ms; below MIN_BYTES the threads cost what they save.
+  static constexpr size_t SLOTS = 3, SLOT = 1u << 20, SLOT_MEDIUM = 2u << 20,
+                          SLOT_LARGE = 4u << 20, MEDIUM = 12u << 20, LARGE = 32u << 20,
+                          MIN_BYTES = 6u << 20, WORKERS = 8;
+  Readback();
   Readback(const Readback &) = delete;
   Readback &operator=(const Readback &) = delete;
   ~Readback();
-  void ensure(size_t slot);
-  // after what is queued on s; returns when out is filled
+  // of a finished array (s has drained past its writers); returns when out is
+  // filled
   void copy(void *out, const void *dev, size_t bytes, hipStream_t s);
 };
 
