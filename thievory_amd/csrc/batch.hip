@@ -16,11 +16,13 @@ namespace {
 constexpr int MBS = 256;
 constexpr int ACC_HASH = 0, ACC_CNT = 64, ACC_LM = 128, RES_HASH = 129, RES_CNT = 193,
               RES_DEPTH = 257, ACC_LONG = 321, ACC_MU = 322, ACC_SCAN_HOST = 323,
-              ACC_SCAN_HBM = 324, ACC_WORDS = 384;
+              ACC_SCAN_HBM = 324, ACC_MF = 325, ACC_WORDS = 384;
 // bottom-up levels: lists up to this length are scanned by one lane, longer
 // ones by a group of BU_G lanes reading BU_R records each per step (measured
 // on the 64-lane R-MAT 25 batch: 8 / 8 / 2 beat 32 / 16 / 2 by 5%; larger
-// steps lose more to reads past the early exit than they save in steps)
+// steps lose more to reads past the early exit than they save in steps; on
+// R-MAT 22 both kernels' levels take 710 us with 8 / 8 / 2, 700 with 8 / 4 / 4,
+// 725 with 4 or 16 / 8 / 2, 740 with 8 / 16 / 2)
 constexpr uint32_t BU_SHORT = 8, BU_G = 8, BU_R = 2;
 // per-wave LDS buffer of long-list vertices, flushed to the global queue with
 // one atomic per flush (an atomic per wave step on one counter serialises)
@@ -32,6 +34,7 @@ struct MsArgs {
   const uint32_t *qc[2];
   const LevelCtr *ctr;
   const uint64_t *eptr;
+  const uint32_t *deg;  // BFS: to sum the next frontier's edges, or null
   const unsigned long long *F;
   unsigned long long *N, *seen;
   uint32_t *nb;
@@ -61,14 +64,15 @@ __global__ void __launch_bounds__(MBS) k_ms_bfs(MsArgs a) {
   __shared__ unsigned long long s_hash[64];
   __shared__ unsigned int s_cnt[64];
   __shared__ uint32_t s_val[64];
-  __shared__ unsigned long long s_lm;
+  __shared__ unsigned long long s_lm, s_mf;
   const uint32_t tid = threadIdx.x;
   if (tid < 64) {
     s_hash[tid] = 0;
     s_cnt[tid] = 0;
     s_val[tid] = a.level + 2 - a.voff[tid];
   }
-  if (tid == 0) s_lm = 0;
+  if (tid == 0) s_lm = s_mf = 0;
+  unsigned long long mf = 0;  // edges of the vertices this lane put on the next frontier
   const ChunkSrc cs = chunk_src(a.ctr, C);
   for (uint32_t c = blockIdx.x; c < cs.total; c += gridDim.x) {
     int q;
@@ -127,7 +131,10 @@ __global__ void __launch_bounds__(MBS) k_ms_bfs(MsArgs a) {
       const uint32_t w = dst[j];
       const unsigned long long gained = gain[j];
       if (!gained) continue;
-      if (on[j] == 0ull) atomicOr(&a.nb[w >> 5], 1u << (w & 31));
+      if (on[j] == 0ull) {
+        atomicOr(&a.nb[w >> 5], 1u << (w & 31));
+        if (a.deg) mf += a.deg[w];
+      }
       atomicOr(&s_lm, gained);
       unsigned long long g = gained;
       while (g) {
@@ -141,12 +148,16 @@ __global__ void __launch_bounds__(MBS) k_ms_bfs(MsArgs a) {
     }
     __syncthreads();
   }
+  if (mf) atomicAdd(&s_mf, mf);
   __syncthreads();
   if (tid < 64 && s_cnt[tid]) {
     atomicAdd(&a.acc[ACC_HASH + tid], s_hash[tid]);
     atomicAdd(&a.acc[ACC_CNT + tid], (unsigned long long)s_cnt[tid]);
   }
-  if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
+  if (tid == 0) {
+    or_new(&a.acc[ACC_LM], s_lm);
+    if (s_mf) atomicAdd(&a.acc[ACC_MF], s_mf);
+  }
 }
 
 // ---- bottom-up BFS levels (symmetric graphs) ---------------------------------
@@ -163,7 +174,6 @@ struct MsBuArgs {
   const uint64_t *eptr;
   const uint32_t *deg;
   const uint32_t *rbit;
-  const uint32_t *fb;           // frontier bitmap: F[v] is read only when v's bit is set
   const unsigned long long *F;
   unsigned long long *N, *seen;
   uint32_t *nb;
@@ -180,7 +190,7 @@ struct MsBuArgs {
 // Per-block digest state for bottom-up levels: lane q of every wave keeps
 // query q's sum and count in registers.
 struct BuDigest {
-  unsigned long long h = 0, scan_host = 0, scan_hbm = 0, mu = 0, lm = 0;
+  unsigned long long h = 0, scan_host = 0, scan_hbm = 0, mu = 0, mf = 0, lm = 0;
   uint32_t cnt = 0;
 };
 
@@ -233,6 +243,7 @@ __device__ __forceinline__ void bu_digest_flush(BuDigest &d, unsigned long long 
   if (d.mu) atomicAdd(&s_misc[1], d.mu);
   if (d.scan_host) atomicAdd(&s_misc[2], d.scan_host);
   if (d.scan_hbm) atomicAdd(&s_misc[3], d.scan_hbm);
+  if (d.mf) atomicAdd(&s_misc[4], d.mf);
   __syncthreads();
   if (tid < 64 && s_cnt[tid]) {
     atomicAdd(&acc[ACC_HASH + tid], s_hash[tid]);
@@ -243,6 +254,22 @@ __device__ __forceinline__ void bu_digest_flush(BuDigest &d, unsigned long long 
     if (s_misc[1]) atomicAdd(&acc[ACC_MU], s_misc[1]);
     if (s_misc[2]) atomicAdd(&acc[ACC_SCAN_HOST], s_misc[2]);
     if (s_misc[3]) atomicAdd(&acc[ACC_SCAN_HBM], s_misc[3]);
+    if (s_misc[4]) atomicAdd(&acc[ACC_MF], s_misc[4]);
+  }
+}
+
+// Frontier masks of R records (0 for absent ones), all loads in flight
+// together.  Straight from F, which is zero off the frontier: asking the
+// frontier bitmap first spared a fifth of the lines and cost a dependent
+// read (64-source BFS, bitmap first / not: R-MAT 20 1.07 / 1.06 ms, 22 1.85 /
+// 1.78, 25 10.4 / 9.9, whose F is larger than the last-level cache).
+template <uint32_t R>
+__device__ __forceinline__ void bu_masks(const MsBuArgs &a, const uint32_t (&v)[R],
+                                         unsigned long long (&f)[R]) {
+#pragma unroll
+  for (uint32_t r = 0; r < R; r++) {
+    f[r] = 0;
+    if (v[r] != 0xFFFFFFFFu) f[r] = a.F[v[r]];
   }
 }
 
@@ -271,8 +298,9 @@ template <int REC>
 __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
   __shared__ unsigned long long s_hash[64];
   __shared__ unsigned int s_cnt[64];
-  __shared__ unsigned long long s_misc[4];
+  __shared__ unsigned long long s_misc[5];
   __shared__ uint32_t s_lq[MBS / 64][BU_LQ];
+  __shared__ uint32_t s_nl[MBS / 64], s_base;
   const uint32_t tid = threadIdx.x, lane = tid & 63;
   uint32_t *my_lq = s_lq[tid >> 6];
   uint32_t nl = 0;  // entries in my_lq (wave-uniform)
@@ -280,7 +308,7 @@ __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
     s_hash[tid] = 0;
     s_cnt[tid] = 0;
   }
-  if (tid < 4) s_misc[tid] = 0;
+  if (tid < 5) s_misc[tid] = 0;
   __syncthreads();
   const uint32_t myval = a.level + 2 - a.voff[lane];
   BuDigest dg;
@@ -317,17 +345,7 @@ __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
           v[j] = 0xFFFFFFFFu;
           if (k + j < d) v[j] = *reinterpret_cast<const uint32_t *>(b + (uint64_t)(k + j) * REC);
         }
-        uint32_t fw[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          fw[j] = 0;
-          if (v[j] != 0xFFFFFFFFu) fw[j] = a.fb[v[j] >> 5];
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          f[j] = 0;
-          if ((fw[j] >> (v[j] & 31)) & 1u) f[j] = a.F[v[j]];
-        }
+        bu_masks<4>(a, v, f);
         acc |= f[0] | f[1] | f[2] | f[3];
         scanned = min(d, k + 4);
         if ((acc & U) == U) break;
@@ -347,6 +365,7 @@ __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
     if (gain) {
       a.N[w] = gain;
       a.seen[w] = sw | gain;
+      dg.mf += d;
     }
     if (!lng && (U & ~gain)) dg.mu += d;
     if (scanned) {
@@ -361,24 +380,42 @@ __global__ void __launch_bounds__(MBS) k_ms_bu(MsBuArgs a) {
     if (a.uval && gain) hw = mix64((w << 32) | a.uval);
     bu_digest_wave(gb, gain, (uint32_t)w, hw, a.uval, myval, lane, a.full, a.n, dg);
   }
-  if (nl) bu_lq_flush(my_lq, nl, a.acc, a.lq, lane);
+  // what is left in the waves' buffers: one atomic a block
+  if (lane == 0) s_nl[tid >> 6] = nl;
+  __syncthreads();
+  uint32_t mine = 0, all = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < MBS / 64; i++) {
+    if (i < (tid >> 6)) mine += s_nl[i];
+    all += s_nl[i];
+  }
+  if (tid == 0 && all) s_base = (uint32_t)atomicAdd(&a.acc[ACC_LONG], (unsigned long long)all);
+  __syncthreads();
+  for (uint32_t i = lane; i < nl; i += 64) a.lq[s_base + mine + i] = my_lq[i];
   bu_digest_flush(dg, a.acc, s_hash, s_cnt, s_misc);
 }
 
 // Long lists: a group of BU_G lanes per queued vertex reads BU_G * BU_R
 // records per step, ORs their frontier masks across the group and stops
-// when every missing lane is found.
+// when every missing lane is found.  Vertices need very different numbers of
+// steps, so a group that is done takes the wave's next vertex at once
+// instead of waiting for the wave's slowest group: a wave loads up to 64
+// queued vertices with their degrees, masks and list addresses (lane i holds
+// vertex i) and hands them out by shuffles.  Bound by the scattered reads of
+// F.  The widest two levels of 64 sources on R-MAT 22: 305 and 145 us with
+// groups that wait, 255 and 134 without waiting, 210 and 118 with the masks
+// read directly (bu_masks).
 template <int REC>
 __global__ void __launch_bounds__(MBS) k_ms_bu_long(MsBuArgs a) {
   __shared__ unsigned long long s_hash[64];
   __shared__ unsigned int s_cnt[64];
-  __shared__ unsigned long long s_misc[4];
+  __shared__ unsigned long long s_misc[5];
   const uint32_t tid = threadIdx.x, lane = tid & 63, sub = tid & (BU_G - 1);
   if (tid < 64) {
     s_hash[tid] = 0;
     s_cnt[tid] = 0;
   }
-  if (tid < 4) s_misc[tid] = 0;
+  if (tid < 5) s_misc[tid] = 0;
   __syncthreads();
   const uint32_t myval = a.level + 2 - a.voff[lane];
   const uint64_t total = a.acc[ACC_LONG];
@@ -386,64 +423,88 @@ __global__ void __launch_bounds__(MBS) k_ms_bu_long(MsBuArgs a) {
   BuDigest dg;
   const uint64_t wave = (uint64_t)blockIdx.x * (MBS / 64) + (tid >> 6);
   const uint64_t nwaves = (uint64_t)gridDim.x * (MBS / 64);
-  for (uint64_t i0 = wave * GPW; i0 < total; i0 += nwaves * GPW) {
-    const uint64_t i = i0 + (lane / BU_G);
-    uint32_t w = 0;
-    unsigned long long U = 0, sw = 0, acc = 0;
-    uint32_t d = 0, scanned = 0;
-    if (i < total) {
-      w = a.lq[i];
-      d = a.deg[w];
-      sw = a.seen[w];
-      U = a.act & ~sw;
-      const unsigned long long b = a.eptr[w];
-      for (uint32_t k = 0; k < d; k += BU_G * BU_R) {
-        uint32_t v[BU_R];
-        unsigned long long f[BU_R];
-#pragma unroll
-        for (uint32_t r = 0; r < BU_R; r++) {
-          const uint32_t e = k + r * BU_G + sub;
-          v[r] = 0xFFFFFFFFu;
-          if (e < d) v[r] = *reinterpret_cast<const uint32_t *>(b + (uint64_t)e * REC);
+  // vertices a wave loads together: its share of a short queue
+  const uint32_t B = (uint32_t)min((uint64_t)64, max((uint64_t)GPW, (total + nwaves - 1) / nwaves));
+  uint64_t i0 = wave * B;             // the next vertices to load
+  uint32_t nxt = 0, have = 0;         // handed out, loaded (wave-uniform)
+  uint32_t bw = 0, bd = 0;            // lane i: loaded vertex i
+  unsigned long long bs = 0, bb = 0;
+  uint32_t w = 0, d = 0, k = 0;       // the group's vertex
+  unsigned long long U = 0, sw = 0, b = 0, acc = 0;
+  bool live = false;
+  for (;;) {
+    const unsigned long long need = __ballot(!live && sub == 0);
+    if (need) {
+      if (nxt >= have && i0 < total) {
+        have = (uint32_t)min((uint64_t)B, total - i0);
+        nxt = 0;
+        if (lane < have) {
+          bw = a.lq[i0 + lane];
+          bd = a.deg[bw];
+          bs = a.seen[bw];
+          bb = a.eptr[bw];
         }
-        uint32_t fw[BU_R];
-#pragma unroll
-        for (uint32_t r = 0; r < BU_R; r++) {
-          fw[r] = 0;
-          if (v[r] != 0xFFFFFFFFu) fw[r] = a.fb[v[r] >> 5];
-        }
-#pragma unroll
-        for (uint32_t r = 0; r < BU_R; r++) {
-          f[r] = 0;
-          if ((fw[r] >> (v[r] & 31)) & 1u) f[r] = a.F[v[r]];
-        }
-        unsigned long long x = f[0];
-#pragma unroll
-        for (uint32_t r = 1; r < BU_R; r++) x |= f[r];
-#pragma unroll
-        for (uint32_t o = BU_G / 2; o; o >>= 1) x |= __shfl_xor(x, o, BU_G);
-        acc |= x;
-        scanned = min(d, k + BU_G * BU_R);
-        if ((acc & U) == U) break;
+        i0 += nwaves * B;
       }
+      const uint32_t slot =
+          nxt + (uint32_t)__popcll(need & ((1ull << (lane & ~(BU_G - 1))) - 1));
+      const uint32_t from = slot & 63;
+      const uint32_t nw = __shfl(bw, from), nd = __shfl(bd, from);
+      const unsigned long long ns = __shfl(bs, from), nb = __shfl(bb, from);
+      if (!live && slot < have) {
+        live = true;
+        w = nw;
+        d = nd;
+        sw = ns;
+        b = nb;
+        U = a.act & ~sw;
+        acc = 0;
+        k = 0;
+      }
+      nxt = min(nxt + (uint32_t)__popcll(need), have);
+      if (!__ballot(live)) break;  // nothing in flight, so nothing was left to hand out
     }
-    const bool leader = sub == 0 && i < total;
+    bool fin = false;
+    if (live) {
+      uint32_t v[BU_R];
+      unsigned long long f[BU_R];
+#pragma unroll
+      for (uint32_t r = 0; r < BU_R; r++) {
+        const uint32_t e = k + r * BU_G + sub;
+        v[r] = 0xFFFFFFFFu;
+        if (e < d) v[r] = *reinterpret_cast<const uint32_t *>(b + (uint64_t)e * REC);
+      }
+      bu_masks<BU_R>(a, v, f);
+      unsigned long long x = f[0];
+#pragma unroll
+      for (uint32_t r = 1; r < BU_R; r++) x |= f[r];
+#pragma unroll
+      for (uint32_t o = BU_G / 2; o; o >>= 1) x |= __shfl_xor(x, o, BU_G);
+      acc |= x;
+      k = min(d, k + BU_G * BU_R);
+      fin = k == d || (acc & U) == U;
+    }
+    const bool leader = fin && sub == 0;
     const unsigned long long gain = acc & U;
     if (leader) {
       if (gain) {
         a.N[w] = gain;
         a.seen[w] = sw | gain;
         atomicOr(&a.nb[w >> 5], 1u << (w & 31));
+        dg.mf += d;
       }
       if (U & ~gain) dg.mu += d;
       const bool hbm = (a.rbit[w >> 5] >> (w & 31)) & 1u;
-      if (hbm) dg.scan_hbm += scanned;
-      else dg.scan_host += scanned;
+      if (hbm) dg.scan_hbm += k;
+      else dg.scan_host += k;
     }
-    unsigned long long hw = 0;
-    if (a.uval && leader && gain) hw = mix64(((unsigned long long)w << 32) | a.uval);
-    bu_digest_wave(__ballot(leader && gain != 0), gain, w, hw, a.uval, myval, lane, a.full, a.n,
-                   dg);
+    if (fin) live = false;
+    const unsigned long long who = __ballot(leader && gain != 0);
+    if (who) {
+      unsigned long long hw = 0;
+      if (a.uval && leader) hw = mix64(((unsigned long long)w << 32) | a.uval);
+      bu_digest_wave(who, gain, w, hw, a.uval, myval, lane, a.full, a.n, dg);
+    }
   }
   bu_digest_flush(dg, a.acc, s_hash, s_cnt, s_misc);
 }
@@ -629,7 +690,7 @@ __global__ void __launch_bounds__(MBS) k_ms_lanebits(const unsigned long long *F
 __global__ void __launch_bounds__(MBS) k_ms_begin(unsigned long long *F, uint32_t *fb,
                                                   uint64_t words, unsigned long long *acc) {
   const uint32_t lane = threadIdx.x & 63;
-  if (blockIdx.x == 0 && threadIdx.x < 5)
+  if (blockIdx.x == 0 && threadIdx.x < 6)
     acc[threadIdx.x < 1 ? ACC_LM : ACC_LONG + threadIdx.x - 1] = 0;
   const uint64_t nw = (uint64_t)gridDim.x * (MBS / 64);
   for (uint64_t w0 = ((uint64_t)blockIdx.x * (MBS / 64) + (threadIdx.x >> 6)) * 64; w0 < words;
@@ -849,6 +910,7 @@ void MultiEngine::launch_level() {
                        full.as<uint32_t>(), n, acc.as<unsigned long long>());
     admit_q.clear();
     mu_est = g.m;  // new lanes miss every vertex
+    mf_known = false;
   }
   level_bu = false;
   if (active) {
@@ -859,24 +921,28 @@ void MultiEngine::launch_level() {
     if (algo == THV_ALGO_BFS && g.sym && g.dir_opt) {
       // direction: the frontier's edges against the edges of the vertices
       // some lane still misses (an upper bound kept since the last
-      // bottom-up level; any admission resets it to m)
-      LevelSide cs;
-      cs.pub_src = c;
-      cs.pub = h_ctr_dev + (level & 1);
-      cs.npub = 1;
-      launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, CMP_COUNT_ONLY, nullptr, 0, 1,
-                     0xFFFFFFFFu, 0, nullptr, 0, nullptr, nullptr, &cs);
-      HIPC(hipStreamSynchronize(stream));
-      const uint64_t mf = h_ctr[level & 1].qw[0] + h_ctr[level & 1].qw[1];
-      level_bu = BU_ALPHA * mf > mu_est && mf > n / 8;
-      // lanes with small frontiers run this level top-down
-      uint64_t td = 0;
-      if (level_bu) {
-        const uint64_t thr = std::max<uint64_t>(1, n / LANE_TD_DIV);
-        for (uint32_t q = 0; q < MAXL; q++)
-          if (((active >> q) & 1ull) && fsz[q] < thr) td |= 1ull << q;
-        if (td == active) level_bu = false;  // every lane's frontier is small
+      // bottom-up level; any admission resets it to m).  The last level has
+      // summed the frontier's edges as it set the frontier's bits; only
+      // admitted sources, which it did not see, make a counting pass and a
+      // wait for its result necessary.
+      uint64_t td = 0;  // lanes with small frontiers run top-down in any case
+      const uint64_t thr = std::max<uint64_t>(1, n / LANE_TD_DIV);
+      for (uint32_t q = 0; q < MAXL; q++)
+        if (((active >> q) & 1ull) && fsz[q] < thr) td |= 1ull << q;
+      const bool counted = td != active && !mf_known;
+      uint64_t mf = mf_next;
+      if (counted) {
+        LevelSide cs;
+        cs.pub_src = c;
+        cs.pub = h_ctr_dev + (level & 1);
+        cs.npub = 1;
+        launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, CMP_COUNT_ONLY, nullptr, 0, 1,
+                       0xFFFFFFFFu, 0, nullptr, 0, nullptr, nullptr, &cs);
+        HIPC(hipStreamSynchronize(stream));
+        mf = h_ctr[level & 1].qw[0] + h_ctr[level & 1].qw[1];
       }
+      level_bu = td != active && BU_ALPHA * mf > mu_est && mf > n / 8;
+      if (!level_bu) td = 0;
       level_td_lanes = level_bu ? td : 0;
       if (level_bu) {
         launch_bottom_up(active & ~td);
@@ -887,7 +953,7 @@ void MultiEngine::launch_level() {
           launch_top_down(c, td);
         }
       } else {
-        launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, CMP_WRITE_ONLY);
+        launch_compact(g, qs, fb[cur].as<uint32_t>(), c, stream, counted ? CMP_WRITE_ONLY : 0);
         launch_top_down(c);
       }
     } else {
@@ -909,7 +975,6 @@ void MultiEngine::launch_bottom_up(uint64_t lanes) {
   b.eptr = g.store.d_eptr.as<uint64_t>();
   b.deg = g.d_deg.as<uint32_t>();
   b.rbit = g.store.d_rbit.as<uint32_t>();
-  b.fb = fb[cur].as<uint32_t>();
   b.F = F[cur].as<unsigned long long>();
   b.N = F[cur ^ 1].as<unsigned long long>();
   b.seen = seen.as<unsigned long long>();
@@ -957,6 +1022,7 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
     }
     a.ctr = c;
     a.eptr = g.store.d_eptr.as<uint64_t>();
+    a.deg = algo == THV_ALGO_BFS && g.sym && g.dir_opt ? g.d_deg.as<uint32_t>() : nullptr;
     a.F = F[cur].as<unsigned long long>();
     a.N = F[cur ^ 1].as<unsigned long long>();
     a.seen = seen.as<unsigned long long>();
@@ -1045,6 +1111,8 @@ void MultiEngine::finish_level(std::vector<LaneResult> &done) {
     stats.host_bytes += h.qw[0] * (uint64_t)g.rec;
     stats.hbm_bytes += h.qw[1] * (uint64_t)g.rec;
   }
+  mf_next = h_acc[ACC_MF];
+  mf_known = true;
   stats.iterations++;
   stats.expand_launches++;
   const uint64_t lm = h_acc[ACC_LM];

@@ -73,6 +73,8 @@ struct MultiEngine {
   // more than n/8 edges (a bottom-up level sweeps all n vertices)
   static constexpr uint64_t BU_ALPHA = 2;
   uint64_t mu_est = 0;
+  uint64_t mf_next = 0;    // edges of the frontier the last level left
+  bool mf_known = false;   // ... and no source was admitted to it since
   bool level_bu = false;
   // Per-lane direction inside a bottom-up level: a lane whose frontier
   // holds fewer than n / LANE_TD_DIV vertices runs top-down (its vertices
