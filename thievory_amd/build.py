@@ -31,7 +31,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}",
           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-Wall", "-Wno-unused-result", "-I", INCLUDE]
 
-LIB_SOURCES = ["graph.cpp", "readback.cpp", "io.cpp", "abi.cpp", "frontier.hip", "expand.hip",
+LIB_SOURCES = ["graph.cpp", "io.cpp", "abi.cpp", "readback.hip", "frontier.hip", "expand.hip",
                "algos.hip", "rmat.hip", "batch.hip", "serve.cpp", "autotune.cpp",
                "bottomup.hip", "cc.hip", "small.hip", "pr.hip", "noalloc.hip", "wide.hip", "probe.hip"]
 CLI_SOURCES = ["cli.cpp"]

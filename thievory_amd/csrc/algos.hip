@@ -439,8 +439,15 @@ static void finish_values(Graph &g, uint32_t *out, thv_stats *st, uint32_t none,
                           bool labels = false) {
   Workspace &w = g.ws;
   if (!out) return;
-  const bool dev = st && !labels && g.n >= COUNT_MIN;
-  if (dev) {
+  uint64_t reached = 0;
+  const bool counted = w.rb.copy(out, w.val.p, g.n * 4, g.stream, none,
+                                 st && !labels ? &reached : nullptr);
+  if (!st) return;
+  if (labels) {
+    st->reached = g.n;
+  } else if (counted) {
+    st->reached = reached;
+  } else if (g.n >= COUNT_MIN) {
     uint32_t *c = reinterpret_cast<uint32_t *>(w.aux.as<unsigned long long>() + AUX_REACHED);
     launch_fill_u32(c, 0u, 2, g.stream);
     hipLaunchKernelGGL(k_count_ne, dim3((uint32_t)std::min<uint64_t>(div_up(g.n, 4096), g.cus)),
@@ -452,12 +459,6 @@ static void finish_values(Graph &g, uint32_t *out, thv_stats *st, uint32_t none,
     ps.xpub = w.h_aux_dev + AUX_REACHED;
     ps.nx = 1;
     launch_publish(ps, g.stream);
-  }
-  w.rb.copy(out, w.val.p, g.n * 4, g.stream);
-  if (!st) return;
-  if (labels) {
-    st->reached = g.n;
-  } else if (dev) {
     HIPC(hipStreamSynchronize(g.stream));
     st->reached = w.h_aux[AUX_REACHED];
   } else {

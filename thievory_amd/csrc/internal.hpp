@@ -81,12 +81,13 @@ struct HostPinned {  // hipHostMalloc'd, mapped into the GPU address space
 };
 
 // Large copies of device arrays to pageable host memory through a ring of
-// pinned slots (readback.cpp).
+// pinned slots (readback.hip).
 struct Readback {
-  // Slots of 4 MB copied 134 MB in 3.0 ms, of 2 MB in 3.5, of 1 MB in 4.4 (an
-  // event wait per slot); smaller arrays take smaller slots, which are as fast
-  // there and allocate less on the process's first copy (6 MB: 1.1 ms).  An 8
-  // MB array gains 0.2 ms; below MIN_BYTES the threads cost what they save.
+  // Slots of 4 MB copy 138 MB in 2.8 ms, of 2 MB in 2.9 (a copy of the runtime
+  // and an event a slot: 3.1); smaller arrays take smaller slots, which are as
+  // fast there and allocate less on the process's first copy (6 MB: 1.1 ms).
+  // A 12 MB array takes 0.34 ms, 0.7 in pageable memory; below MIN_BYTES the
+  // threads cost what they save.
   static constexpr size_t SLOTS = 3, SLOT = 1u << 20, SLOT_MEDIUM = 2u << 20,
                           SLOT_LARGE = 4u << 20, MEDIUM = 12u << 20, LARGE = 32u << 20,
                           MIN_BYTES = 6u << 20, WORKERS = 8;
@@ -95,8 +96,10 @@ struct Readback {
   Readback &operator=(const Readback &) = delete;
   ~Readback();
   // of a finished array (s has drained past its writers); returns when out is
-  // filled
-  void copy(void *out, const void *dev, size_t bytes, hipStream_t s);
+  // filled.  True if *count (may be null) holds the number of 32-bit words
+  // that differ from none: large arrays only
+  bool copy(void *out, const void *dev, size_t bytes, hipStream_t s, uint32_t none = 0,
+            uint64_t *count = nullptr);
 };
 
 // ---- store -------------------------------------------------------------------
