@@ -534,6 +534,7 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   const uint32_t L = a.L;
   const bool lane_ok = lane < L;
   if (tid == 0) s_lm = 0;
+  unsigned long long lm = 0;  // lanes this wave improved somewhere
   const ChunkSrc cs = chunk_src(a.ctr, C);
   for (uint32_t c = blockIdx.x; c < cs.total; c += gridDim.x) {
     int q;
@@ -571,11 +572,10 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
       // row is still a valid distance; an improved source is in N anyway)
       uint32_t kprev = 0xFFFFFFFFu, dprev = 0;
       bool mprev = false;
+      uint32_t blo = 0, bhi = 0;  // lane j: the lanes that edge g0 + j improved
       for (uint32_t j0 = 0; j0 < cnt; j0 += 8) {
-        uint32_t w[8], dv[8], dw[8], wt[8];
-        bool on[8];
-        uint32_t kk[8], ds[8];
-        bool nw[8], ms[8];
+        uint32_t w[8], dw[8], wt[8], kk[8], ds[8];
+        bool on[8], nw[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           const uint32_t jj = min(j0 + j, cnt - 1);
@@ -584,27 +584,19 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
           kk[j] = __builtin_amdgcn_readlane(my_k, jj);
           nw[j] = kk[j] != (j ? kk[j - 1] : kprev);  // a new source (uniform)
         }
-        // the new sources' lane masks, then their rows, all in flight together
+        // the new sources' lane masks, then their rows and the destinations',
+        // all in flight together
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-          ms[j] = false;
-          if (nw[j]) ms[j] = lane_ok && ((s_m[kk[j]] >> lane) & 1ull);
+          if (nw[j]) mprev = lane_ok && ((s_m[kk[j]] >> lane) & 1ull);
+          on[j] = j0 + j < cnt && mprev;
         }
+        kprev = kk[7];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           ds[j] = 0u;
-          if (nw[j] && ms[j]) ds[j] = a.dist[(uint64_t)s_v[kk[j]] * L + lane];
+          if (nw[j] && on[j]) ds[j] = a.dist[(uint64_t)s_v[kk[j]] * L + lane];
         }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          if (nw[j]) {
-            mprev = ms[j];
-            dprev = ds[j];
-          }
-          on[j] = j0 + j < cnt && mprev;
-          dv[j] = dprev;
-        }
-        kprev = kk[7];
 #pragma unroll
         for (int j = 0; j < 8; j++) dw[j] = on[j] ? a.dist[(uint64_t)w[j] * L + lane] : 0u;
         // An improvement is judged against the row just read, so the
@@ -612,35 +604,32 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
         // together.  A lane whose atomicMin loses to a smaller concurrent
         // write is marked anyway: that write lowered dist[w] in this level
         // and marks the same (w, lane), so the next frontier is unchanged.
-        unsigned long long b[8], old[8];
 #pragma unroll
         for (int j = 0; j < 8; j++) {
+          if (nw[j]) dprev = ds[j];
           bool imp = false;
           if (on[j]) {
-            const unsigned long long nd = (unsigned long long)dv[j] + wt[j];
+            const unsigned long long nd = (unsigned long long)dprev + wt[j];
             if (nd < dw[j]) {
               imp = true;
               atomicMin(&a.dist[(uint64_t)w[j] * L + lane], (uint32_t)nd);
             }
           }
-          b[j] = __ballot(imp);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          old[j] = ~0ull;
-          if (b[j] && lane == 0) old[j] = atomicOr(&a.N[w[j]], b[j]);
-        }
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-          if (b[j] && lane == 0) {
-            if (old[j] == 0ull) atomicOr(&a.nb[w[j] >> 5], 1u << (w[j] & 31));
-            atomicOr(&s_lm, b[j]);
+          const unsigned long long b = __ballot(imp);
+          lm |= b;
+          if (lane == j0 + j) {
+            blo = (uint32_t)b;
+            bhi = (uint32_t)(b >> 32);
           }
         }
       }
+      // the marks of all 64 edges at once, a lane each
+      const unsigned long long b = ((unsigned long long)bhi << 32) | blo;
+      if (b && atomicOr(&a.N[my_w], b) == 0ull) atomicOr(&a.nb[my_w >> 5], 1u << (my_w & 31));
     }
     __syncthreads();
   }
+  if (lane == 0 && lm) atomicOr(&s_lm, lm);
   __syncthreads();
   if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
 }
