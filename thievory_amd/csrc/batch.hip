@@ -509,19 +509,23 @@ __global__ void __launch_bounds__(MBS) k_ms_bu_long(MsBuArgs a) {
   bu_digest_flush(dg, a.acc, s_hash, s_cnt, s_misc);
 }
 
-// SSSP: lane q of a wave relaxes query q.  A wave owns 64 consecutive
-// work-space edges at a time: each lane loads one record (coalesced) and
-// ranks it once; the wave then walks the 64 edges, broadcasting each with
-// readlane, with the source and destination distance rows of 8 edges in
-// flight before the first compare.
+// SSSP: a group of G lanes relaxes an edge, lane q of the group query q.  A
+// wave owns 64 consecutive work-space edges at a time: each lane loads one
+// record (coalesced) and ranks it once.  With G = 64 the wave then walks the
+// 64 edges, broadcasting each with readlane, with the source and destination
+// distance rows of 8 edges in flight before the first compare; the rows bound
+// it (64 sources on R-MAT 20: some 4.7 TB/s of them on the widest levels).
+// Batches of fewer queries take 8, 4 or 2 edges at once instead of idle
+// lanes, ms a call on R-MAT 20 with G = 64 / the least that holds them: 1
+// source 2.8 / 1.4, 8 4.4 / 1.9, 16 5.0 / 2.5, 32 5.3 / 3.6.
 // Chunks of 1,024 edges (4 waves x 4 x 64), or of 256 where a level has too
 // few to fill the chip with those: a wave's edges are a serial chain (64 take
-// 20 us, 256 80).  Batches of 64 sources, ms a call with 1,024 / 256 only:
-// R-MAT 14 2.18 / 1.39, 20 8.24 / 7.96, 22 24.6 / 25.7; so 256 below 8 large
-// chunks per CU.
+// 20 us, 256 80).  Batches of 64 sources, ms a call with 1,024 / 256 only
+// (some of each since saved elsewhere): R-MAT 14 2.18 / 1.39, 20
+// 8.24 / 7.96, 22 24.6 / 25.7; so 256 below 8 large chunks per CU.
 constexpr uint32_t SSSP_C = 256, SSSP_LARGE = 1024;
 
-template <uint32_t C>
+template <uint32_t C, uint32_t G>
 __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   constexpr uint32_t NW = C / 32;
   constexpr uint32_t WAVES = MBS / 64, PER_WAVE = C / WAVES;
@@ -532,9 +536,10 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   __shared__ unsigned long long s_lm;
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const uint32_t L = a.L;
-  const bool lane_ok = lane < L;
+  const uint32_t sub = lane & (G - 1), eg = lane / G;
+  const bool lane_ok = sub < L;
   if (tid == 0) s_lm = 0;
-  unsigned long long lm = 0;  // lanes this wave improved somewhere
+  unsigned long long lm = 0;  // lanes (of all groups) improved somewhere
   const ChunkSrc cs = chunk_src(a.ctr, C);
   for (uint32_t c = blockIdx.x; c < cs.total; c += gridDim.x) {
     int q;
@@ -567,12 +572,42 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
         my_w = r.x;
         my_wt = r.y;
       }
+      uint32_t blo = 0, bhi = 0;  // lane j: the queries that edge g0 + j improved
+      if (G < 64) {
+        constexpr uint32_t EPS = 64 / G;  // edges at once
+        for (uint32_t j0 = 0; j0 * EPS < cnt; j0 += 8) {
+          uint32_t w[8], wt[8], ds[8], dw[8];
+          bool on[8];
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            const uint32_t e = (j0 + j) * EPS + eg;
+            w[j] = __shfl(my_w, e);
+            wt[j] = __shfl(my_wt, e);
+            const uint32_t k = __shfl(my_k, e);
+            on[j] = e < cnt && lane_ok && ((s_m[k] >> sub) & 1ull);
+            ds[j] = on[j] ? a.dist[(uint64_t)s_v[k] * L + sub] : 0u;
+            dw[j] = on[j] ? a.dist[(uint64_t)w[j] * L + sub] : 0u;
+          }
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            const unsigned long long nd = (unsigned long long)ds[j] + wt[j];
+            const bool imp = on[j] && nd < dw[j];
+            if (imp) atomicMin(&a.dist[(uint64_t)w[j] * L + sub], (uint32_t)nd);
+            const unsigned long long b = __ballot(imp);
+            lm |= b;
+            if (lane / EPS == j0 + j)
+              blo = (uint32_t)(b >> (lane % EPS * G)) & (uint32_t)((1ull << (G & 63)) - 1);
+          }
+        }
+        if (blo && atomicOr(&a.N[my_w], (unsigned long long)blo) == 0ull)
+          atomicOr(&a.nb[my_w >> 5], 1u << (my_w & 31));
+        continue;
+      }
       // consecutive edges mostly share their source: its lane mask and
       // distance row are read once per source, not once per edge (a stale
       // row is still a valid distance; an improved source is in N anyway)
       uint32_t kprev = 0xFFFFFFFFu, dprev = 0;
       bool mprev = false;
-      uint32_t blo = 0, bhi = 0;  // lane j: the lanes that edge g0 + j improved
       for (uint32_t j0 = 0; j0 < cnt; j0 += 8) {
         uint32_t w[8], dw[8], wt[8], kk[8], ds[8];
         bool on[8], nw[8];
@@ -629,9 +664,19 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
     }
     __syncthreads();
   }
+  for (uint32_t o = 32; o >= G; o >>= 1) lm |= lm >> o;
+  if (G < 64) lm &= (1ull << (G & 63)) - 1;
   if (lane == 0 && lm) atomicOr(&s_lm, lm);
   __syncthreads();
   if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
+}
+
+template <uint32_t C>
+void launch_sssp(const MsArgs &a, uint32_t grid, hipStream_t s) {
+  if (a.L <= 8) hipLaunchKernelGGL((k_ms_sssp<C, 8>), dim3(grid), dim3(MBS), 0, s, a);
+  else if (a.L <= 16) hipLaunchKernelGGL((k_ms_sssp<C, 16>), dim3(grid), dim3(MBS), 0, s, a);
+  else if (a.L <= 32) hipLaunchKernelGGL((k_ms_sssp<C, 32>), dim3(grid), dim3(MBS), 0, s, a);
+  else hipLaunchKernelGGL((k_ms_sssp<C, 64>), dim3(grid), dim3(MBS), 0, s, a);
 }
 
 struct AdmitArgs {
@@ -1051,10 +1096,8 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
       const uint32_t C = large ? SSSP_LARGE : SSSP_C;
       const uint64_t chunks = div_up(h.qw[0], C) + div_up(h.qw[1], C);
       const uint64_t sg = std::max<uint64_t>(1, std::min<uint64_t>(chunks, 1u << 30));
-      if (large)
-        hipLaunchKernelGGL(k_ms_sssp<SSSP_LARGE>, dim3((uint32_t)sg), dim3(MBS), 0, stream, a);
-      else
-        hipLaunchKernelGGL(k_ms_sssp<SSSP_C>, dim3((uint32_t)sg), dim3(MBS), 0, stream, a);
+      if (large) launch_sssp<SSSP_LARGE>(a, (uint32_t)sg, stream);
+      else launch_sssp<SSSP_C>(a, (uint32_t)sg, stream);
     }
     HIPC(hipGetLastError());
   }

@@ -161,7 +161,14 @@ bool Readback::copy(void *out, const void *dev, size_t bytes, hipStream_t s, uin
     return false;
   }
   const size_t slot = bytes >= LARGE ? SLOT_LARGE : bytes >= MEDIUM ? SLOT_MEDIUM : SLOT;
-  std::unique_ptr<Ring> held = RingPool::get().take(SLOTS * slot);
+  std::unique_ptr<Ring> held;
+  try {
+    held = RingPool::get().take(SLOTS * slot);
+  } catch (const std::exception &) {  // no pinned memory to be had: the plain copy
+    (void)hipGetLastError();
+    HIPC(hipMemcpy(out, dev, bytes, hipMemcpyDeviceToHost));
+    return false;
+  }
   Ring &r = *held;
   const size_t chunks = div_up(bytes, slot);
   std::atomic<size_t> ready{0};             // chunks [0, ready) are in their slots

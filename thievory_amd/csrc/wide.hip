@@ -32,7 +32,7 @@
 // its value and the winner appends its segments to the next queue; CC and
 // SSSP lower values with atomicMin and append a vertex the first time it
 // improves in a level (a stamp per vertex holds the last level that queued
-// it).  Appends are wave-aggregated.
+// it).  Appends go out block by block, through LDS.
 #include <algorithm>
 
 #include <rocprim/device/device_radix_sort.hpp>
