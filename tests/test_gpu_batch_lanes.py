@@ -17,7 +17,7 @@ def _check(g, og, srcs):
         assert (r["hash"][i], r["reached"][i], r["depth"][i]) == tuple(want), (len(srcs), i, s)
 
 
-@pytest.mark.parametrize("k", [1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 64])
+@pytest.mark.parametrize("k", [1, 2, 7, 8, 9, 15, 16, 17, 31, 32, 33, 34, 47, 62, 63, 64])
 def test_lanes_an_edge(k):
     print("case: batch SSSP of", k, flush=True)
     rng = np.random.default_rng(k)
@@ -30,7 +30,7 @@ def test_lanes_an_edge(k):
         _check(g, og, srcs[::-1].copy())
 
 
-@pytest.mark.parametrize("k", [3, 12, 20])
+@pytest.mark.parametrize("k", [3, 12, 20, 33, 34])
 def test_large_chunks(k):
     print("case: batch SSSP large chunks", k, flush=True)
     og = O.rmat(18, 24, seed=9, weights=True)

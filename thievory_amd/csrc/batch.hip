@@ -509,23 +509,41 @@ __global__ void __launch_bounds__(MBS) k_ms_bu_long(MsBuArgs a) {
   bu_digest_flush(dg, a.acc, s_hash, s_cnt, s_misc);
 }
 
+// Bits of x at the even places of 64.
+__device__ __forceinline__ unsigned long long spread_bits(uint32_t x) {
+  unsigned long long v = x;
+  v = (v | (v << 16)) & 0x0000FFFF0000FFFFull;
+  v = (v | (v << 8)) & 0x00FF00FF00FF00FFull;
+  v = (v | (v << 4)) & 0x0F0F0F0F0F0F0F0Full;
+  v = (v | (v << 2)) & 0x3333333333333333ull;
+  v = (v | (v << 1)) & 0x5555555555555555ull;
+  return v;
+}
+
 // SSSP: a group of G lanes relaxes an edge, lane q of the group query q.  A
 // wave owns 64 consecutive work-space edges at a time: each lane loads one
-// record (coalesced) and ranks it once.  With G = 64 the wave then walks the
-// 64 edges, broadcasting each with readlane, with the source and destination
-// distance rows of 8 edges in flight before the first compare; the rows bound
-// it (64 sources on R-MAT 20: some 4.7 TB/s of them on the widest levels).
-// Batches of fewer queries take 8, 4 or 2 edges at once instead of idle
-// lanes, ms a call on R-MAT 20 with G = 64 / the least that holds them: 1
-// source 2.8 / 1.4, 8 4.4 / 1.9, 16 5.0 / 2.5, 32 5.3 / 3.6.
+// record (coalesced) and ranks it once; the groups then take the 64 edges in
+// turn, SSSP_U each in flight.  Bound by the distance rows (64 sources on R-MAT
+// 20: 75M edges of two 256-byte rows, one of them mostly in L1).
+// - Up to 32 queries: 8, 4 or 2 edges at once instead of idle lanes, ms a call
+//   on R-MAT 20 with a whole wave an edge / the least group that holds them: 1
+//   source 2.8 / 1.3, 8 4.4 / 1.8, 16 5.0 / 2.4, 32 5.3 / 3.4.
+// - More, an even number (rows then start at 8-byte addresses): PAIR, two
+//   queries a lane and two edges at once, half the load instructions.  64
+//   sources on R-MAT 14 1.09 -> 1.05, 20 5.76 -> 4.81, 22 18.6 -> 15.5.
+// - More, an odd number: a wave an edge.  Its edges are broadcast with
+//   readlane, and a source's row is read once per run of its edges.
+// SSSP_U: 8 need 103 registers and 2 hide too little (R-MAT 20, 64 sources, with
+// 2 / 4 / 8: 5.1 / 4.8 / 5.3 ms).
 // Chunks of 1,024 edges (4 waves x 4 x 64), or of 256 where a level has too
 // few to fill the chip with those: a wave's edges are a serial chain (64 take
 // 20 us, 256 80).  Batches of 64 sources, ms a call with 1,024 / 256 only
-// (some of each since saved elsewhere): R-MAT 14 2.18 / 1.39, 20
-// 8.24 / 7.96, 22 24.6 / 25.7; so 256 below 8 large chunks per CU.
+// (some of each since saved elsewhere): R-MAT 14 2.18 / 1.39, 20 8.24 / 7.96,
+// 22 24.6 / 25.7; so 256 below 8 large chunks per CU.
+constexpr uint32_t SSSP_U = 4;
 constexpr uint32_t SSSP_C = 256, SSSP_LARGE = 1024;
 
-template <uint32_t C, uint32_t G>
+template <uint32_t C, uint32_t G, bool PAIR = false>
 __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   constexpr uint32_t NW = C / 32;
   constexpr uint32_t WAVES = MBS / 64, PER_WAVE = C / WAVES;
@@ -537,7 +555,8 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   const uint32_t tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const uint32_t L = a.L;
   const uint32_t sub = lane & (G - 1), eg = lane / G;
-  const bool lane_ok = sub < L;
+  const bool lane_ok = PAIR ? 2 * sub < L : sub < L;
+  unsigned long long lm1 = 0;  // PAIR: the odd queries' (lm: the even ones')
   if (tid == 0) s_lm = 0;
   unsigned long long lm = 0;  // lanes (of all groups) improved somewhere
   const ChunkSrc cs = chunk_src(a.ctr, C);
@@ -573,13 +592,53 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
         my_wt = r.y;
       }
       uint32_t blo = 0, bhi = 0;  // lane j: the queries that edge g0 + j improved
+      if (PAIR) {
+        // lane q of 32 takes queries 2q and 2q + 1 of one of two edges
+        uint32_t be = 0, bo = 0;  // lane j: edge g0 + j's even and odd queries
+        for (uint32_t j0 = 0; j0 * 2 < cnt; j0 += SSSP_U) {
+          uint32_t w[SSSP_U], wt[SSSP_U], m[SSSP_U];
+          uint2 ds[SSSP_U], dw[SSSP_U];
+#pragma unroll
+          for (int j = 0; j < (int)SSSP_U; j++) {
+            const uint32_t e = (j0 + j) * 2 + eg;
+            w[j] = __shfl(my_w, e);
+            wt[j] = __shfl(my_wt, e);
+            const uint32_t k = __shfl(my_k, e);
+            m[j] = e < cnt && lane_ok ? (uint32_t)(s_m[k] >> (2 * sub)) & 3u : 0u;
+            ds[j] = dw[j] = make_uint2(0, 0);
+            if (m[j]) {
+              ds[j] = *reinterpret_cast<const uint2 *>(&a.dist[(uint64_t)s_v[k] * L + 2 * sub]);
+              dw[j] = *reinterpret_cast<const uint2 *>(&a.dist[(uint64_t)w[j] * L + 2 * sub]);
+            }
+          }
+#pragma unroll
+          for (int j = 0; j < (int)SSSP_U; j++) {
+            const unsigned long long n0 = (unsigned long long)ds[j].x + wt[j];
+            const unsigned long long n1 = (unsigned long long)ds[j].y + wt[j];
+            const bool i0 = (m[j] & 1u) && n0 < dw[j].x, i1 = (m[j] & 2u) && n1 < dw[j].y;
+            uint32_t *p = &a.dist[(uint64_t)w[j] * L + 2 * sub];
+            if (i0) atomicMin(p, (uint32_t)n0);
+            if (i1) atomicMin(p + 1, (uint32_t)n1);
+            const unsigned long long b0 = __ballot(i0), b1 = __ballot(i1);
+            lm |= b0;
+            lm1 |= b1;
+            if (lane / 2 == j0 + j) {
+              be = (uint32_t)(b0 >> ((lane & 1) * 32));
+              bo = (uint32_t)(b1 >> ((lane & 1) * 32));
+            }
+          }
+        }
+        const unsigned long long b = spread_bits(be) | (spread_bits(bo) << 1);
+        if (b && atomicOr(&a.N[my_w], b) == 0ull) atomicOr(&a.nb[my_w >> 5], 1u << (my_w & 31));
+        continue;
+      }
       if (G < 64) {
         constexpr uint32_t EPS = 64 / G;  // edges at once
-        for (uint32_t j0 = 0; j0 * EPS < cnt; j0 += 8) {
-          uint32_t w[8], wt[8], ds[8], dw[8];
-          bool on[8];
+        for (uint32_t j0 = 0; j0 * EPS < cnt; j0 += SSSP_U) {
+          uint32_t w[SSSP_U], wt[SSSP_U], ds[SSSP_U], dw[SSSP_U];
+          bool on[SSSP_U];
 #pragma unroll
-          for (int j = 0; j < 8; j++) {
+          for (int j = 0; j < (int)SSSP_U; j++) {
             const uint32_t e = (j0 + j) * EPS + eg;
             w[j] = __shfl(my_w, e);
             wt[j] = __shfl(my_wt, e);
@@ -589,7 +648,7 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
             dw[j] = on[j] ? a.dist[(uint64_t)w[j] * L + sub] : 0u;
           }
 #pragma unroll
-          for (int j = 0; j < 8; j++) {
+          for (int j = 0; j < (int)SSSP_U; j++) {
             const unsigned long long nd = (unsigned long long)ds[j] + wt[j];
             const bool imp = on[j] && nd < dw[j];
             if (imp) atomicMin(&a.dist[(uint64_t)w[j] * L + sub], (uint32_t)nd);
@@ -666,6 +725,7 @@ __global__ void __launch_bounds__(MBS) k_ms_sssp(MsArgs a) {
   }
   for (uint32_t o = 32; o >= G; o >>= 1) lm |= lm >> o;
   if (G < 64) lm &= (1ull << (G & 63)) - 1;
+  if (PAIR) lm = spread_bits((uint32_t)lm) | (spread_bits((uint32_t)(lm1 | lm1 >> 32)) << 1);
   if (lane == 0 && lm) atomicOr(&s_lm, lm);
   __syncthreads();
   if (tid == 0) or_new(&a.acc[ACC_LM], s_lm);
@@ -676,6 +736,8 @@ void launch_sssp(const MsArgs &a, uint32_t grid, hipStream_t s) {
   if (a.L <= 8) hipLaunchKernelGGL((k_ms_sssp<C, 8>), dim3(grid), dim3(MBS), 0, s, a);
   else if (a.L <= 16) hipLaunchKernelGGL((k_ms_sssp<C, 16>), dim3(grid), dim3(MBS), 0, s, a);
   else if (a.L <= 32) hipLaunchKernelGGL((k_ms_sssp<C, 32>), dim3(grid), dim3(MBS), 0, s, a);
+  else if (a.L % 2 == 0)
+    hipLaunchKernelGGL((k_ms_sssp<C, 32, true>), dim3(grid), dim3(MBS), 0, s, a);
   else hipLaunchKernelGGL((k_ms_sssp<C, 64>), dim3(grid), dim3(MBS), 0, s, a);
 }
 
