@@ -468,7 +468,7 @@ def pr_block(T, O, args):
         t0 = time.perf_counter()
         r, st = g.pr(mode)
         wall = time.perf_counter() - t0
-        s = step_summary([st], wall, f"k_expand<PR_{mode.upper()}>")
+        s = step_summary([st], wall, f"k_pr_{mode}")
         s["vertices"], s["edges"] = g.n, g.m
         s["store"], s["tuning"] = g.store_info(), tuning
         out[mode] = s
