@@ -198,8 +198,11 @@ __global__ void __launch_bounds__(CBS) k_tcount(CompactArgs a) {
   }
 }
 
-constexpr int SBS = 1024;
-constexpr int SNW = SBS / 64;
+// Threads of the segments' block: one a segment up to 256 (2^26 vertices),
+// 1,024 past that.  A block of 1,024 starts only on a CU with half of its
+// wave slots free: beside another stream's SSSP level (a server's) it waited
+// 2 ms on average, and the scan itself gains nothing from idle waves.
+constexpr int SBS_FEW = 256, SBS = 1024;
 
 // Segment bases: the count kernels add each tile's four sums (entries and
 // edges per queue) into its segment of SEG tiles; one block scans the
@@ -207,10 +210,11 @@ constexpr int SNW = SBS / 64;
 // counters and clears the segment sums for the next count.  A tile's base
 // is its segment's base plus the tiles before it in the segment, which the
 // write pass adds itself (one coalesced load).
+template <int BS>
 __device__ __forceinline__ void sscan_block(const CompactArgs &a) {
-  __shared__ unsigned long long sh[4][SNW + 1];
+  __shared__ unsigned long long sh[4][BS / 64 + 1];
   unsigned long long carry[4] = {0, 0, 0, 0};
-  for (uint32_t b = 0; b < a.nseg; b += SBS) {
+  for (uint32_t b = 0; b < a.nseg; b += BS) {
     const uint32_t sg = b + threadIdx.x;
     unsigned long long x[4] = {0, 0, 0, 0};
     if (sg < a.nseg) {
@@ -223,7 +227,7 @@ __device__ __forceinline__ void sscan_block(const CompactArgs &a) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       unsigned long long tot;
-      const unsigned long long ex = block_excl_scan<SBS>(x[i], sh[i], &tot);
+      const unsigned long long ex = block_excl_scan<BS>(x[i], sh[i], &tot);
       if (sg < a.nseg) a.sbase[sg * 4 + i] = carry[i] + ex;
       carry[i] += tot;
     }
@@ -248,11 +252,15 @@ __device__ __forceinline__ void sscan_block(const CompactArgs &a) {
   }
 }
 
-__global__ void __launch_bounds__(SBS) k_sscan(CompactArgs a) { sscan_block(a); }
+template <int BS>
+__global__ void __launch_bounds__(BS) k_sscan(CompactArgs a) {
+  sscan_block<BS>(a);
+}
 
 // Both tile-table sets of a probe in one launch: block k scans set k.
-__global__ void __launch_bounds__(SBS) k_sscan2(CompactArgs a0, CompactArgs a1) {
-  sscan_block(blockIdx.x ? a1 : a0);
+template <int BS>
+__global__ void __launch_bounds__(BS) k_sscan2(CompactArgs a0, CompactArgs a1) {
+  sscan_block<BS>(blockIdx.x ? a1 : a0);
 }
 
 // Base of a tile: its segment's base plus the tiles before it in the
@@ -1238,7 +1246,8 @@ void launch_compact(Graph &g, QueueSet &w, const uint32_t *front, LevelCtr *ctr,
   // the tile bases and totals are still in place
   if (!(mode & CMP_WRITE_ONLY)) {
     hipLaunchKernelGGL(k_tcount, dim3(grid), dim3(CBS), 0, s, a);
-    hipLaunchKernelGGL(k_sscan, dim3(1), dim3(SBS), 0, s, a);
+    if (a.nseg <= SBS_FEW) hipLaunchKernelGGL(k_sscan<SBS_FEW>, dim3(1), dim3(SBS_FEW), 0, s, a);
+    else hipLaunchKernelGGL(k_sscan<SBS>, dim3(1), dim3(SBS), 0, s, a);
   }
   if (!(mode & CMP_COUNT_ONLY)) {
     hipLaunchKernelGGL(k_twrite, dim3(grid), dim3(CBS), 0, s, a);
@@ -1340,7 +1349,9 @@ void launch_bu_probe(Graph &g, QueueSet &w, const uint32_t *front, uint32_t *vis
     a.nseg = (uint32_t)div_up(a.ntiles, SEG);
     a.ctr = k == 0 ? cs : cl;
   }
-  hipLaunchKernelGGL(k_sscan2, dim3(2), dim3(SBS), 0, s, sa2[0], sa2[1]);
+  if (sa2[0].nseg <= SBS_FEW)
+    hipLaunchKernelGGL(k_sscan2<SBS_FEW>, dim3(2), dim3(SBS_FEW), 0, s, sa2[0], sa2[1]);
+  else hipLaunchKernelGGL(k_sscan2<SBS>, dim3(2), dim3(SBS), 0, s, sa2[0], sa2[1]);
   LbaseArgs lb;
   lb.lcnt = p.lcnt;
   lb.sbase = w.sbase[1].as<unsigned long long>();
