@@ -1143,9 +1143,9 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
         else hipLaunchKernelGGL((k_ms_bfs<4, 8>), dim3(grid), dim3(MBS), 0, stream, a);
       }
     } else {
-      // One block per chunk, not a persistent grid: an SSSP level runs for
-      // milliseconds, and short blocks let the work-groups of other streams
-      // (a BFS cohort's levels) take CUs as they free up.  The chunk count
+      // One block per chunk, not a persistent grid, unless room is to be left:
+      // an SSSP level runs for milliseconds, and short blocks let the
+      // work-groups of other streams take CUs as they free up.  The chunk count
       // comes from the compaction just launched (one readback).
       LevelSide ps;
       ps.pub_src = c;
@@ -1157,7 +1157,8 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
       const bool large = h.qw[0] + h.qw[1] >= 8ull * g.cus * SSSP_LARGE;
       const uint32_t C = large ? SSSP_LARGE : SSSP_C;
       const uint64_t chunks = div_up(h.qw[0], C) + div_up(h.qw[1], C);
-      const uint64_t sg = std::max<uint64_t>(1, std::min<uint64_t>(chunks, 1u << 30));
+      const uint64_t most = leave_room ? (uint64_t)ROOM_BPC * g.cus : 1u << 30;
+      const uint64_t sg = std::max<uint64_t>(1, std::min<uint64_t>(chunks, most));
       if (large) launch_sssp<SSSP_LARGE>(a, (uint32_t)sg, stream);
       else launch_sssp<SSSP_C>(a, (uint32_t)sg, stream);
     }

@@ -63,6 +63,10 @@ struct Server {
   // saturated at R-MAT 25).
   static constexpr int COHORT_ENGINES = 4;
   static constexpr double SPILL_MS = 10.0;
+  // SSSP levels leave room (MultiEngine::leave_room) while BFS queries come:
+  // one may arrive during a level that was launched with none waiting
+  static constexpr double BFS_RECENT_MS = 1000.0;
+  double last_bfs = -2 * BFS_RECENT_MS;
 
   double now_ms() const { return (now_ns() - t0) * 1e-6; }
   void loop();
@@ -114,11 +118,13 @@ void Server::loop() {
             waiting[a].pop_front();
             e.admit(r.src, r.ticket);
             res[r.ticket].start_ms = now_ms();
+            if (a == 0) last_bfs = res[r.ticket].start_ms;
           }
         }
       }
       for (size_t i = 0; i < eng.size(); i++)
         if (!inflight[i] && eng[i]->busy()) {
+          eng[i]->leave_room = now_ms() - last_bfs < BFS_RECENT_MS;
           eng[i]->launch_level();
           inflight[i] = 1;
         }
