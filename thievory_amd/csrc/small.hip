@@ -159,6 +159,9 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
   }
   __syncthreads();
   uint32_t nfar = s.fars, levels = 0, lv = a.level_value, stamp = a.stamp;
+  // without a near vertex the loop starts with the bucket step, which resets
+  // s.fars: every wave has its copy first
+  __syncthreads();
   uint64_t left = a.unvisited;
   // this thread's share of the totals over all levels
   unsigned long long tn = 0, te[2] = {0, 0}, tt = 0, last = 0;
