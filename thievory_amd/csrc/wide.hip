@@ -611,6 +611,15 @@ constexpr uint32_t CTR_Q = 0, CTR_FOUND = 32, CTR_DIGEST = 48, CTR_EDGES = 64;
 static void ensure_work(Graph64 &g) {
   const uint64_t qcap = g.k + (g.m >> g.seg_shift) + 1;
   if (g.val.p) return;
+  // The ids of a graph are bounded by the memory their n values would take:
+  // they are never all there, but CC's digest visits every id (2^60 of them
+  // would take years).
+  size_t fr = 0, tot = 0;
+  drop_idle_engines();
+  HIPC(hipMemGetInfo(&fr, &tot));
+  if (g.n > fr / 8)
+    fail(THV_ENOMEM, "the values of " + std::to_string(g.n) + " vertices exceed the " +
+                         std::to_string(fr) + " bytes of free device memory");
   for (auto &q : g.q) q.alloc(qcap * 8);
   g.ctr.alloc((CTR_EDGES + g.cus) * 8);
   g.stamp.alloc(std::max<uint64_t>(g.N, 1) * 4);
