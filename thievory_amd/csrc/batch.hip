@@ -928,7 +928,9 @@ MultiEngine::~MultiEngine() {
 uint64_t MultiEngine::bytes_needed(const Graph &g, int algo, uint32_t lanes, bool keep_full) {
   const uint64_t n = g.n, words = bitmap_words(n);
   uint64_t b = 2 * (words * 4 + (n + 1) * 8);                       // fb, F
-  b += 2 * ((n + 1) * 12) + 2 * (g.m / QC_MIN + 2) * 4;              // queues
+  // queues (a table of one chunk start per 1,024 edges, as callers' budgets were
+  // chosen for; the finer one in use takes 0.02 bytes an edge more)
+  b += 2 * ((n + 1) * 12) + 2 * (g.m / 1024 + 2) * 4;
   b += (n / TILE + 1) * TILE * 4;                                     // long-list queue
   if (algo == THV_ALGO_BFS)
     b += (n + 1) * 8 + words * 4 + (keep_full ? (uint64_t)lanes * n * 4 : 0);
