@@ -189,7 +189,7 @@ void build_parent_hints(Graph &g) {
   hipLaunchKernelGGL(k_hint_finish, dim3(grid ? grid : 1), dim3(BBS), 0, s,
                      key.as<unsigned long long>(), g.n, g.store.d_hint.as<uint32_t>());
   HIPC(hipGetLastError());
-  HIPC(hipStreamSynchronize(s));
+  g.store.hints_meet = hint_trees_meet(g, s);  // (waits for the stream)
 }
 
 }  // namespace thv
