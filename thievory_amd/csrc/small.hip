@@ -50,29 +50,83 @@ struct SmallShared {
   uint32_t cnt, over, fars, lo, any;
 };
 
+// One thread's vertices and edges of the frontier left in the bitmap (host,
+// HBM): summed once at the end, since LDS adds to one address take turns.
+struct Left {
+  uint32_t nf[2] = {0, 0};
+  unsigned long long mf[2] = {0, 0};
+};
+
+// Runs of lanes whose ids share a bitmap word.  One CU's atomics on one word
+// take turns, 7-8 ns each (on different words 0.7-2): a sorted list of
+// consecutive ids is best sent as one atomic a run (BFS from the hub of a star
+// of 20,000 leaves: 298 us in this kernel with an atomic a leaf, 50 so; leaves
+// spread over 4M ids 87 either way).
+struct Runs {
+  bool few;             // few enough runs to be worth the shuffles (wave-uniform)
+  uint32_t start, end;  // this lane's run
+};
+__device__ __forceinline__ Runs runs_of(uint32_t word) {
+  const uint32_t lane = lane_id(), before = __shfl_up(word, 1, 64);
+  const unsigned long long heads = wave_ballot(lane == 0 || word != before);
+  const unsigned long long upto = heads & (~0ull >> (63 - lane));
+  const unsigned long long after = heads & ~(~0ull >> (63 - lane));
+  Runs r;
+  r.few = __popcll(heads) <= 16;
+  r.start = 63 - __builtin_clzll(upto);
+  r.end = after ? (uint32_t)__builtin_ctzll(after) - 1 : 63u;
+  return r;
+}
+// OR of x over the lanes of the run up to this one.
+__device__ __forceinline__ uint32_t run_or(uint32_t x, const Runs &r) {
+  const uint32_t lane = lane_id();
+#pragma unroll
+  for (uint32_t d = 1; d < 64; d <<= 1) {
+    const uint32_t y = __shfl_up(x, d, 64);
+    if (lane >= r.start + d) x |= y;
+  }
+  return x;
+}
+
+// The vertices of the lanes with `on` to the bitmap (BFS: counted).  Every
+// lane of the wave takes part.
+template <bool VAL>
+__device__ __forceinline__ void leave(const SmallArgs &a, Left &left, bool on, uint32_t w) {
+  const Runs r = runs_of(on ? w >> 5 : 0xFFFFFFFFu);
+  uint32_t bits = on ? 1u << (w & 31) : 0u;
+  bool send = on;
+  if (r.few) {
+    bits = run_or(bits, r);
+    send = on && lane_id() == r.end;
+  }
+  if (send) atomicOr(&a.front[w >> 5], bits);
+  if (VAL || !on) return;
+  const uint32_t d = a.deg[w];
+  const bool hbm = !a.split || ((a.rbit[w >> 5] >> (w & 31)) & 1u);
+  left.nf[0] += d && !hbm;
+  left.nf[1] += d && hbm;
+  left.mf[0] += hbm ? 0u : d;
+  left.mf[1] += hbm ? d : 0u;
+}
+
 // Appends (w, nv) for the lanes with `take`; past the queue's capacity the
 // vertex goes to the bitmap and the block ends after this level.
 template <bool VAL>
-__device__ __forceinline__ void push(const SmallArgs &a, SmallShared &s, bool take, uint32_t w,
-                                     uint32_t nv) {
+__device__ __forceinline__ void push(const SmallArgs &a, SmallShared &s, Left &left, bool take,
+                                     uint32_t w, uint32_t nv) {
   const unsigned long long b = wave_ballot(take);
   if (!b) return;
   uint32_t at = 0;
   if (lane_id() == 0) at = atomicAdd(&s.cnt, (uint32_t)__popcll(b));
   at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + lanes_below(b);
-  if (!take) return;
-  if (at < QCAP) {
+  if (take && at < QCAP) {
     s.id[at] = w;
     if (VAL) s.nval[at] = nv;
-  } else {
-    s.over = 1;
-    atomicOr(&a.front[w >> 5], 1u << (w & 31));
-    const uint32_t d = a.deg[w], q = a.split ? (a.rbit[w >> 5] >> (w & 31)) & 1u : 1u;
-    if (d) {
-      atomicAdd(&s.sum[q], 1ull);
-      atomicAdd(&s.sum[2 + q], (unsigned long long)d);
-    }
   }
+  const bool out = take && at >= QCAP;
+  if (!wave_ballot(out)) return;
+  if (out) s.over = 1;
+  leave<VAL>(a, left, out, w);
 }
 
 // Appends (w, nv) to the far list `to` (counted in s.fars).
@@ -117,6 +171,7 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
   unsigned long long state = 0;
   const uint32_t count = a.list ? *a.count : 1u;
   bool refused = false;
+  Left rest;
   if (a.list && count > (FAR ? a.far_cap : QCAP)) {
     refused = true;
   } else if (!a.list) {
@@ -150,7 +205,7 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
         // the top-down loop leaves a frontier's level to its compaction
         if (!VAL && in) a.val[v] = a.level_value - 1;
         const bool near = in && (!FAR || x < thr);
-        push<VAL>(a, s, near, v, x);
+        push<VAL>(a, s, rest, near, v, x);
         if (FAR) push_far(a, s, fin, in && !near, v, x);
       }
       __syncthreads();
@@ -187,7 +242,7 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
         const unsigned long long x = i < nfar ? fin[i] : 0ull;
         const uint32_t w = (uint32_t)x, nv = (uint32_t)(x >> 32);
         const bool cur = i < nfar && ld_agent(&a.val[w]) == nv;
-        push<VAL>(a, s, cur && nv < thr, w, nv);
+        push<VAL>(a, s, rest, cur && nv < thr, w, nv);
         push_far(a, s, fout, cur && nv >= thr, w, nv);
       }
       __syncthreads();
@@ -306,26 +361,51 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
       }
       uint32_t old[UNR];
       if (ALGO == A_BFS) {
-        // a wide level tests the word first; a narrow one is bound by the
-        // latency of that test
+        // A narrow level is bound by the latency of its steps; a wide one tests
+        // the word first and sends one atomic for a run of lanes on one word
+        // (its last lane's, with the run's bits; a lane's bit that an earlier
+        // lane of the run has too is that lane's).
+        bool won[UNR];
         if (Eu > SB) {
+          Runs r[UNR];
+          uint32_t mine[UNR];  // few runs: the bits of the run's earlier lanes
 #pragma unroll
           for (uint32_t j = 0; j < UNR; j++)
             old[j] = w[j] != 0xFFFFFFFFu ? a.vis[w[j] >> 5] : 0xFFFFFFFFu;
+#pragma unroll
+          for (uint32_t j = 0; j < UNR; j++) {
+            const uint32_t bit = 1u << (w[j] & 31);
+            won[j] = !(old[j] & bit);
+            r[j] = runs_of(w[j] >> 5);
+            uint32_t bits = won[j] ? bit : 0u;
+            bool send = won[j];
+            mine[j] = 0;
+            if (r[j].few) {
+              bits = run_or(bits, r[j]);
+              mine[j] = __shfl_up(bits, 1, 64);
+              if (lane == r[j].start) mine[j] = 0;
+              send = lane == r[j].end && bits;
+            }
+            if (send) old[j] = atomicOr(&a.vis[w[j] >> 5], bits);
+          }
+#pragma unroll
+          for (uint32_t j = 0; j < UNR; j++) {
+            if (r[j].few) old[j] = __shfl(old[j], r[j].end, 64) | mine[j];
+            won[j] = won[j] && !(old[j] & (1u << (w[j] & 31)));
+          }
         } else {
 #pragma unroll
-          for (uint32_t j = 0; j < UNR; j++) old[j] = w[j] != 0xFFFFFFFFu ? 0u : 0xFFFFFFFFu;
+          for (uint32_t j = 0; j < UNR; j++) {
+            old[j] = 0xFFFFFFFFu;
+            if (w[j] != 0xFFFFFFFFu) old[j] = atomicOr(&a.vis[w[j] >> 5], 1u << (w[j] & 31));
+          }
+#pragma unroll
+          for (uint32_t j = 0; j < UNR; j++) won[j] = !(old[j] & (1u << (w[j] & 31)));
         }
 #pragma unroll
         for (uint32_t j = 0; j < UNR; j++) {
-          const uint32_t bit = 1u << (w[j] & 31);
-          if (!(old[j] & bit)) old[j] = atomicOr(&a.vis[w[j] >> 5], bit);
-        }
-#pragma unroll
-        for (uint32_t j = 0; j < UNR; j++) {
-          const bool won = !(old[j] & (1u << (w[j] & 31)));
-          if (won) a.val[w[j]] = lv;
-          push<VAL>(a, s, won, w[j], 0);
+          if (won[j]) a.val[w[j]] = lv;
+          push<VAL>(a, s, rest, won[j], w[j], 0);
         }
       } else {
 #pragma unroll
@@ -338,7 +418,7 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
         for (uint32_t j = 0; j < UNR; j++) {
           const bool won = x[j] < old[j];
           const bool near = won && (!FAR || x[j] < thr);
-          push<VAL>(a, s, near, w[j], x[j]);
+          push<VAL>(a, s, rest, near, w[j], x[j]);
           if (FAR) push_far(a, s, fin, won && !near, w[j], x[j]);
         }
       }
@@ -360,15 +440,9 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
   // vertex is there through its newer entry)
   __syncthreads();
   if (state) {
-    for (uint32_t i = tid; i < F; i += SB) {
-      const uint32_t id = s.id[i];
-      if (VAL && ld_agent(&a.val[id]) != s.nval[i]) continue;
-      atomicOr(&a.front[id >> 5], 1u << (id & 31));
-      const uint32_t d = a.deg[id], q = a.split ? (a.rbit[id >> 5] >> (id & 31)) & 1u : 1u;
-      if (d) {
-        atomicAdd(&s.sum[q], 1ull);
-        atomicAdd(&s.sum[2 + q], (unsigned long long)d);
-      }
+    for (uint32_t i = tid; i < (F + SB - 1) / SB * SB; i += SB) {
+      const uint32_t id = i < F ? s.id[i] : 0u;
+      leave<VAL>(a, rest, i < F && (!VAL || ld_agent(&a.val[id]) == s.nval[i]), id);
     }
     if (FAR) {
       for (uint32_t i = tid; i < nfar; i += SB) {
@@ -382,6 +456,17 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
   te[0] = wave_sum(te[0]);
   te[1] = wave_sum(te[1]);
   tt = wave_sum(tt);
+  if (state && !VAL) {
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const uint32_t nf = wave_sum(rest.nf[i]);
+      const unsigned long long mf = wave_sum(rest.mf[i]);
+      if (lane == 0 && nf) {
+        atomicAdd(&s.sum[i], (unsigned long long)nf);
+        atomicAdd(&s.sum[2 + i], mf);
+      }
+    }
+  }
   if (lane == 0) {
     if (tn) atomicAdd(&s.sum[5], tn);
     if (te[0]) atomicAdd(&s.sum[6], te[0]);
