@@ -239,6 +239,18 @@ static bool small_frontier(uint64_t nf, uint64_t mf, Algo algo = A_BFS) {
   return nf <= SPARSE_MAX && mf <= (algo == A_SSSP ? SMALL_EDGES_SSSP : SMALL_EDGES);
 }
 
+// A frontier's edges as k_small weighs them: BFS, host records twice.
+static uint64_t small_weight(Algo algo, uint64_t host, uint64_t hbm) {
+  return (algo == A_BFS ? 2 * host : host) + hbm;
+}
+static uint64_t small_weight(Graph &g, Algo algo, uint32_t src) {
+  const uint64_t d = g.h_off[src + 1] - g.h_off[src];
+  const Store &t = g.store;
+  const size_t p = std::upper_bound(t.pv.begin(), t.pv.end(), src) - t.pv.begin() - 1;
+  const bool hbm = t.pres[p] != 0;
+  return small_weight(algo, hbm ? 0 : d, hbm ? d : 0);
+}
+
 // Levels from the frontier {src} (from_src: its bit alone is set in
 // `front`) or from the one the bitmap holds, run by k_small until the
 // frontier is empty or too large; returns after the stream has drained.
@@ -283,6 +295,8 @@ static SmallOut run_small(Graph &g, Workspace &w, Algo algo, uint32_t *front, bo
       edge_max, algo == A_SSSP ? SMALL_EDGES_SSSP : SMALL_EDGES);
   a.ratio = ratio;
   a.unvisited = unvisited;
+  a.new_max = g.n > SMALL_NEW ? SMALL_NEW : UINT64_MAX;
+  a.edges = g.m;
   a.max_levels = SMALL_LEVELS;
   const bool mapped = w.h_aux_dev != nullptr;
   a.out = reinterpret_cast<SmallOut *>((mapped ? w.h_aux_dev : aux) + AUX_SMALL);
@@ -352,7 +366,9 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st, bool fr
   int cur = 0;
   double expand_ms = 0;
   uint32_t launches = 0;
-  bool small = from_src;  // the frontier is known or likely to be small
+  // the frontier is known or likely to be small
+  bool small = from_src && small_frontier(1, small_weight(g, algo, src), algo);
+  from_src = small;
   SmallTry tries;
   const uint64_t t0 = now_ns();
   for (uint32_t L = 0;; L++) {
@@ -400,7 +416,8 @@ static void value_loop(Graph &g, Workspace &w, Algo algo, thv_stats *st, bool fr
     if (h.qn[0] + h.qn[1] == 0) break;
     stats_level(g, st, h);
     cur ^= 1;
-    small = small_frontier(h.qn[0] + h.qn[1], h.qw[0] + h.qw[1], algo) && tries.ready();
+    small = small_frontier(h.qn[0] + h.qn[1], small_weight(algo, h.qw[0], h.qw[1]), algo) &&
+            tries.ready();
   }
   if (st) {
     st->ms = (now_ns() - t0) * 1e-6;
@@ -565,10 +582,11 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
   // HBM side of a top-down level: tiles with frontier vertices taken as nf
   // vertices over the tiles at random
   auto td_hbm_cost = [&](uint64_t nf, uint64_t mf) {
-    if (small_frontier(nf, mf)) return SMALL_FIXED + (double)mf * SMALL_NS_EDGE * 1e-9;
     const double tiles_work = ntiles_d * -std::expm1(-(double)nf / ntiles_d);
-    return TD_FIXED + ((double)nf * TD_NS_ENTRY + (double)mf * TD_NS_EDGE +
-                       ntiles_d * TD_NS_TILE_ALL + tiles_work * TD_NS_TILE) * 1e-9;
+    const double chip = TD_FIXED + ((double)nf * TD_NS_ENTRY + (double)mf * TD_NS_EDGE +
+                                    ntiles_d * TD_NS_TILE_ALL + tiles_work * TD_NS_TILE) * 1e-9;
+    if (!small_frontier(nf, mf)) return chip;
+    return std::min(chip, SMALL_FIXED + (double)mf * SMALL_NS_EDGE * 1e-9);
   };
   auto list_cost = [&]() { return (double)last_cand * LIST_NS_CAND * 1e-9 + LIST_FIXED; };
   uint64_t visited_edges = 0, prev_nf = 0;
@@ -805,11 +823,10 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
       launch_compact(g, w.qs, front, c, s, CMP_COUNT_ONLY, w.val.as<uint32_t>(), L + 1, 1,
                      0xFFFFFFFFu, 0, nullptr, 0, nullptr, nullptr, &cs);
     }
-    if (quick && d0 <= small_edges((double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED)) {
+    const uint64_t small_first = small_edges((double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED);
+    if (quick && small_weight(g, A_BFS, src) <= small_first) {
       // one small list: this level and the small ones after it in one launch
-      if (small_run(L, true, small_edges((double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED),
-                    g.m, nullptr))
-        break;
+      if (small_run(L, true, small_first, g.m, nullptr)) break;
       fused_next = small_left = true;
       L += (uint32_t)small_levels - 1;  // none: level 0 again, its sums known
       continue;
@@ -910,7 +927,8 @@ static void bfs_direction_optimizing(Graph &g, uint32_t src, thv_stats *st) {
     }
     const uint64_t small_max =
         small_edges(cand < 0 ? (double)g.n * PROBE_NS_VERTEX * 1e-9 + PROBE_FIXED : list_cost());
-    if (!bu && !probed && !resumed && nf <= SPARSE_MAX && mf <= small_max) {
+    if (!bu && !probed && !resumed && nf <= SPARSE_MAX &&
+        small_weight(A_BFS, h.qw[0], h.qw[1]) <= small_max) {
       LevelSide zs;
       zs.zero = clear;
       zs.nzero = clear ? words : 0;
@@ -1110,7 +1128,8 @@ static void sssp_delta(Graph &g, uint32_t src, thv_stats *st) {
   unsigned long long *aux = w.aux.as<unsigned long long>();
   uint32_t *d_min = reinterpret_cast<uint32_t *>(aux + AUX_MIN);
   launch_fill_u32(d_min, 0xFFFFFFFFu, 2, s);
-  bool from_src = true, small = true;  // the pending set is {src}
+  // the pending set is {src}
+  bool small = small_frontier(1, small_weight(g, A_SSSP, src), A_SSSP), from_src = small;
   SmallTry tries;
   const uint64_t t0 = now_ns();
   for (uint32_t it = 0;; it++) {

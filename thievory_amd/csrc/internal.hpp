@@ -420,7 +420,15 @@ void launch_list_front(Graph &g, const uint32_t *front, uint32_t *list, uint32_t
 // 32,768 0.149, 131,072 0.153; scale 16 0.320 / 0.313 / 0.322.  SSSP edges
 // take an atomicMin and an 8-byte record: scale 14 0.51 / 0.51 / 0.47, scale
 // 16 1.12 / 1.13 / 1.21, scale 20 2.66 / 2.87 / 2.88.
+// BFS: a host record counts as two, since one CU's reads over the link do not
+// fill it (random graph, 65,536 vertices of degree 32, its lists on the host,
+// ms with all counted as one / so / by the general path alone 0.64 / 0.51 /
+// 0.56); and, all edges in HBM, a level that would find more than SMALL_NEW
+// vertices is left too: they cost 1.5-3 ns each and their queue does not hold
+// them (the same graph in HBM 0.42 / 0.37 / 0.38; a star of 20,000 leaves in
+// k_small 0.13, by the general path 0.17).
 constexpr uint32_t SMALL_EDGES = 32768, SMALL_EDGES_SSSP = 16384;
+constexpr uint32_t SMALL_NEW = 16384;
 constexpr uint32_t SMALL_LEVELS = 4096;  // levels per launch (it then resumes from the bitmap)
 struct SmallOut {
   unsigned long long state;     // 0 the frontier is empty, 1 the bitmap holds the rest,
@@ -452,6 +460,8 @@ struct SmallArgs {
   uint32_t edge_max, max_levels;
   double ratio;                 // BFS, > 0: a level also ends the run when its edges x ratio
   uint64_t unvisited;           //   exceed the edges left (unvisited before the first level)
+  uint64_t new_max, edges;      // BFS: or when it would find more than new_max vertices, of its
+                                //   edges the unvisited share of the graph's
   SmallOut *out;
 };
 void launch_small(Graph &g, Algo algo, const SmallArgs &a, hipStream_t s);

@@ -23,7 +23,8 @@
 //
 // The block gives up (and the general path takes over) when a frontier has
 // more than SPARSE_MAX vertices (its LDS holds 24 bytes of each) or SMALL_EDGES
-// edges: past that the chip finishes a level sooner than one CU does.
+// edges, or would find more than SMALL_NEW vertices: past that the chip
+// finishes a level sooner than one CU does.
 #include "internal.hpp"
 #include "scan.hpp"
 
@@ -300,7 +301,22 @@ __global__ void __launch_bounds__(SB) k_small(SmallArgs a) {
       break;
     }
     left -= min<uint64_t>(left, E);
-    if (E > a.edge_max || levels == a.max_levels ||
+    bool wide = E > a.edge_max ||
+                (ALGO == A_BFS && (double)E * (double)left > (double)a.new_max * (double)a.edges);
+    if (ALGO == A_BFS && a.split && !wide && 2 * E > a.edge_max) {  // host records count twice
+      unsigned long long eh = 0;
+      for (uint32_t i = tid; i < F; i += SB) {
+        const uint32_t id = s.id[i], d = (i + 1 < F ? s.pre[i + 1] : (uint32_t)E) - s.pre[i];
+        if (d && !((a.rbit[id >> 5] >> (id & 31)) & 1u)) eh += d;
+      }
+      eh = wave_sum(eh);
+      if (lane == 0 && eh) atomicAdd(&s.sum[9], eh);
+      __syncthreads();
+      wide = E + s.sum[9] > a.edge_max;
+      __syncthreads();
+      if (tid == 0) s.sum[9] = 0;
+    }
+    if (wide || levels == a.max_levels ||
         (a.ratio > 0 && (double)E * a.ratio > (double)left)) {
       state = 1;
       break;
