@@ -36,6 +36,7 @@
 #include <algorithm>
 
 #include <rocprim/device/device_radix_sort.hpp>
+#include <rocprim/device/device_select.hpp>
 
 #include "internal.hpp"
 #include "scan.hpp"
@@ -423,38 +424,64 @@ Graph64::~Graph64() {
   if (h_ctr) (void)hipHostFree(h_ctr);
 }
 
+// The n keys of a, sorted, each once, to b (n places); a is scratch.  Returns
+// how many.  count: a device word.
+static uint64_t sorted_unique(uint64_t *a, uint64_t *b, uint64_t n, unsigned long long *count,
+                              DevMem &tmp, hipStream_t s) {
+  rocprim::double_buffer<uint64_t> db(a, b);
+  size_t bytes = 0, ubytes = 0;
+  HIPC(rocprim::radix_sort_keys(nullptr, bytes, db, (size_t)n, 0u, 64u, s));
+  HIPC(rocprim::unique(nullptr, ubytes, a, b, count, (size_t)n, rocprim::equal_to<uint64_t>(), s));
+  bytes = std::max(bytes, ubytes);
+  if (tmp.bytes < bytes) tmp.alloc(bytes);
+  HIPC(rocprim::radix_sort_keys(tmp.p, bytes, db, (size_t)n, 0u, 64u, s));
+  HIPC(rocprim::unique(tmp.p, bytes, db.current(), db.alternate(), count, (size_t)n,
+                       rocprim::equal_to<uint64_t>(), s));
+  unsigned long long u = 0;
+  HIPC(hipMemcpyAsync(&u, count, 8, hipMemcpyDeviceToHost, s));
+  if (db.alternate() != b)
+    HIPC(hipMemcpyAsync(b, db.alternate(), n * 8, hipMemcpyDeviceToDevice, s));
+  HIPC(hipStreamSynchronize(s));
+  return u;
+}
+
 // Numbers the destinations and writes the records (in mapped pinned host
 // memory): pieces of the array go to the GPU, which finds each destination
-// among the listed ids; those of a piece that are not listed come back
-// sorted and are merged into `extra`, and the piece is numbered again once
-// extra is complete.
+// among the listed ids.  Those of a piece that are not listed are sorted and
+// made unique there and merged into `extra`; such a piece's records are written
+// once extra is complete.
 static void number_destinations(Graph64 &g, const uint64_t *dst, const uint32_t *w) {
   constexpr uint64_t PIECE = 16ull << 20;
   const uint64_t piece = std::max<uint64_t>(1, std::min(PIECE, g.m));
   hipStream_t s = g.stream;
-  DevMem d_dst, d_w, d_rec, d_miss, d_miss2, d_n, tmp, d_extra;
-  d_dst.alloc(piece * 8);
-  if (w) d_w.alloc(piece * 4);
-  d_rec.alloc(piece * g.rec);
-  d_miss.alloc(piece * 8);
-  d_n.alloc(8);
-  std::vector<uint64_t> extra;
+  // destinations, missing ones, weights, counts of missing and of unique ones
+  const uint64_t at_miss = piece * 8, at_n = at_miss + piece * 8, at_w = at_n + 16;
+  DevMem buf, keys, tmp, extra;
+  uint64_t x = 0;  // ids in extra
+  buf.alloc(at_w + (w ? piece * 4 : 0));
+  unsigned char *b = buf.as<unsigned char>();
+  uint64_t *d_dst = reinterpret_cast<uint64_t *>(b);
+  uint64_t *d_miss = reinterpret_cast<uint64_t *>(b + at_miss);
+  unsigned long long *d_n = reinterpret_cast<unsigned long long *>(b + at_n);
+  uint32_t *d_w = w ? reinterpret_cast<uint32_t *>(b + at_w) : nullptr;
   std::vector<uint8_t> again(div_up(std::max<uint64_t>(g.m, 1), piece), 0);
-  unsigned char *rec = static_cast<unsigned char *>(g.h_edges.p);
+  unsigned char *rec = static_cast<unsigned char *>(g.h_edges.dev);
   const int grid = grid_of(piece, 16 * g.cus);
+  uint64_t held = UINT64_MAX;  // the piece that is in the buffer
+  // writes a piece's records; how many of its destinations are missing
   auto number = [&](uint64_t e0, uint64_t cnt, bool final) {
-    HIPC(hipMemcpyAsync(d_dst.p, dst + e0, cnt * 8, hipMemcpyHostToDevice, s));
-    if (w) HIPC(hipMemcpyAsync(d_w.p, w + e0, cnt * 4, hipMemcpyHostToDevice, s));
-    launch_fill_u32(d_n.as<uint32_t>(), 0u, 2, s);
-    hipLaunchKernelGGL(k_wide_number, dim3(grid), dim3(WBS), 0, s, d_dst.as<uint64_t>(),
-                       w ? d_w.as<uint32_t>() : nullptr, cnt, g.d_uid.as<uint64_t>(), g.k,
-                       final ? d_extra.as<uint64_t>() : nullptr, (uint64_t)extra.size(), g.rec,
-                       d_rec.as<unsigned char>(), d_miss.as<uint64_t>(),
-                       d_n.as<unsigned long long>());
+    if (held != e0) {
+      HIPC(hipMemcpyAsync(d_dst, dst + e0, cnt * 8, hipMemcpyHostToDevice, s));
+      if (w) HIPC(hipMemcpyAsync(d_w, w + e0, cnt * 4, hipMemcpyHostToDevice, s));
+      held = e0;
+    }
+    launch_fill_u32(reinterpret_cast<uint32_t *>(d_n), 0u, 2, s);
+    hipLaunchKernelGGL(k_wide_number, dim3(grid), dim3(WBS), 0, s, d_dst, d_w, cnt,
+                       g.d_uid.as<uint64_t>(), g.k, final ? extra.as<uint64_t>() : nullptr, x, g.rec,
+                       rec + e0 * g.rec, d_miss, d_n);
     HIPC(hipGetLastError());
     unsigned long long n = 0;
-    HIPC(hipMemcpyAsync(rec + e0 * g.rec, d_rec.p, cnt * g.rec, hipMemcpyDeviceToHost, s));
-    HIPC(hipMemcpyAsync(&n, d_n.p, 8, hipMemcpyDeviceToHost, s));
+    HIPC(hipMemcpyAsync(&n, d_n, 8, hipMemcpyDeviceToHost, s));
     HIPC(hipStreamSynchronize(s));
     return (uint64_t)n;
   };
@@ -462,36 +489,35 @@ static void number_destinations(Graph64 &g, const uint64_t *dst, const uint32_t 
     const uint64_t n = number(e0, std::min(piece, g.m - e0), false);
     if (!n) continue;
     again[e0 / piece] = 1;
-    if (!d_miss2.p) d_miss2.alloc(piece * 8);
-    rocprim::double_buffer<uint64_t> db(d_miss.as<uint64_t>(), d_miss2.as<uint64_t>());
-    size_t bytes = 0;
-    HIPC(rocprim::radix_sort_keys(nullptr, bytes, db, (size_t)n, 0u, 64u, s));
-    if (tmp.bytes < bytes) tmp.alloc(bytes);
-    HIPC(rocprim::radix_sort_keys(tmp.p, bytes, db, (size_t)n, 0u, 64u, s));
-    std::vector<uint64_t> found(n), both;
-    HIPC(hipMemcpyAsync(found.data(), db.current(), n * 8, hipMemcpyDeviceToHost, s));
-    HIPC(hipStreamSynchronize(s));
-    found.erase(std::unique(found.begin(), found.end()), found.end());
-    both.reserve(extra.size() + found.size());
-    std::set_union(extra.begin(), extra.end(), found.begin(), found.end(),
-                   std::back_inserter(both));
-    extra.swap(both);
+    if (keys.bytes < n * 8) keys.alloc(n * 8);
+    const uint64_t u = sorted_unique(d_miss, keys.as<uint64_t>(), n, d_n + 1, tmp, s);
+    if (!x) {
+      extra.swap(keys);
+      x = u;
+    } else {  // with those of earlier pieces
+      DevMem both;
+      both.alloc((x + u) * 8);
+      uint64_t *p = both.as<uint64_t>();
+      HIPC(hipMemcpyAsync(p, extra.p, x * 8, hipMemcpyDeviceToDevice, s));
+      HIPC(hipMemcpyAsync(p + x, keys.p, u * 8, hipMemcpyDeviceToDevice, s));
+      HIPC(hipStreamSynchronize(s));
+      if (extra.bytes < (x + u) * 8) extra.alloc((x + u) * 8);
+      x = sorted_unique(p, extra.as<uint64_t>(), x + u, d_n + 1, tmp, s);
+    }
   }
-  g.N = g.k + extra.size();
+  g.N = g.k + x;
   if (g.N > ITEM_MASK) fail(THV_ENOTSUP, "more than 2^40 vertices with edges");
-  if (!extra.empty()) {
-    d_extra.alloc(extra.size() * 8);
-    HIPC(hipMemcpy(d_extra.p, extra.data(), extra.size() * 8, hipMemcpyHostToDevice));
-    for (uint64_t e0 = 0; e0 < g.m; e0 += piece)
-      if (again[e0 / piece]) number(e0, std::min(piece, g.m - e0), true);
-    DevMem uid;
-    uid.alloc(g.N * 8);
-    if (g.k) HIPC(hipMemcpy(uid.p, g.d_uid.p, g.k * 8, hipMemcpyDeviceToDevice));
-    HIPC(hipMemcpy(uid.as<uint64_t>() + g.k, d_extra.p, extra.size() * 8,
-                   hipMemcpyDeviceToDevice));
-    g.d_uid.swap(uid);
-  }
-  g.h_extra.swap(extra);
+  if (!x) return;
+  DevMem uid;
+  uid.alloc(g.N * 8);
+  if (g.k) HIPC(hipMemcpyAsync(uid.p, g.d_uid.p, g.k * 8, hipMemcpyDeviceToDevice, s));
+  HIPC(hipMemcpyAsync(uid.as<uint64_t>() + g.k, extra.p, x * 8, hipMemcpyDeviceToDevice, s));
+  for (uint64_t e0 = 0; e0 < g.m; e0 += piece)
+    if (again[e0 / piece]) number(e0, std::min(piece, g.m - e0), true);
+  g.h_extra.resize(x);
+  HIPC(hipMemcpyAsync(g.h_extra.data(), extra.p, x * 8, hipMemcpyDeviceToHost, s));
+  HIPC(hipStreamSynchronize(s));
+  g.d_uid.swap(uid);
 }
 
 Graph64 *graph64_from_lists(uint64_t n, uint64_t k, const uint64_t *ids, const uint64_t *loff,
