@@ -189,7 +189,8 @@ void build_parent_hints(Graph &g) {
   hipLaunchKernelGGL(k_hint_finish, dim3(grid ? grid : 1), dim3(BBS), 0, s,
                      key.as<unsigned long long>(), g.n, g.store.d_hint.as<uint32_t>());
   HIPC(hipGetLastError());
-  g.store.hints_meet = hint_trees_meet(g, s);  // (waits for the stream)
+  HIPC(hipStreamSynchronize(s));
+  g.store.hints_meet = -1;
 }
 
 }  // namespace thv

@@ -174,12 +174,13 @@ int grid_for(uint64_t n, int cap) {
 
 }  // namespace
 
-// From a sample: whether the lists outside the giant tree of hints hold no more
-// records than two of every list in HBM, which are what CC reads instead (a
-// record takes some 50-70 ps either way).  Random graph of degree 8, 2^20
-// vertices, device ms from the hints / from two records: in HBM 0.78 / 0.32,
-// half of it 0.90 / 0.29; R-MAT 23, edge factor 32, 0.25 / 0.53.
-bool hint_trees_meet(Graph &g, hipStream_t s) {
+// From a sample, once for the hints of a store: whether the lists outside the
+// giant tree of hints hold no more records than two of every list in HBM,
+// which are what CC reads instead (a record takes some 50-70 ps either way).
+// Random graph of degree 8, 2^20 vertices, device ms from the hints / from two
+// records: in HBM 0.78 / 0.32, half of it 0.90 / 0.29; R-MAT 23, edge factor 32,
+// 0.25 / 0.53.
+static bool hint_trees_meet(Graph &g, hipStream_t s) {
   DevMem &buf = g.ws.qs.slist;
   static_assert(CC_SAMPLES * sizeof(HintSample) <= TILE * 4, "a tile holds the sample");
   if (buf.bytes < CC_SAMPLES * sizeof(HintSample)) fail(THV_ESTATE, "sample buffer too small");
@@ -219,7 +220,8 @@ bool cc_union_find(Graph &g, thv_stats *st) {
   const uint64_t *eptr = g.store.d_eptr.as<uint64_t>();
   const uint32_t *deg = g.d_deg.as<uint32_t>(), *rbit = g.store.d_rbit.as<uint32_t>();
   const uint32_t *hint = g.store.d_hint.as<uint32_t>();  // null without hints
-  const bool by_hint = hint && g.store.hints_meet;
+  if (hint && g.store.hints_meet < 0) g.store.hints_meet = hint_trees_meet(g, s);
+  const bool by_hint = hint && g.store.hints_meet > 0;
   hipLaunchKernelGGL(k_cc_start, dim3(grid), dim3(UBS), 0, s, comp, by_hint ? hint : nullptr, n);
   const int lgrid = grid_for(n, 4 * g.cus);  // ends with an atomic per block
   if (by_hint) {

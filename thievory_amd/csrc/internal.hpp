@@ -127,7 +127,7 @@ struct Store {
   // bytes out of the budget; a resident store holds them beside the lists.
   bool hint_reserved = false;
   DevMem d_hint;
-  bool hints_meet = false;           // the hints form a giant tree (hint_trees_meet)
+  int hints_meet = -1;               // the hints form a giant tree; -1: not looked yet (CC does)
   bool sparse_first = false;         // residency ranked sparsest partitions first
 };
 
@@ -514,7 +514,6 @@ void run_cc(Graph &g, uint32_t *out, thv_stats *st);
 // cc.hip: components of a symmetric graph into ws.val; false when a link
 // hit its step guard (the caller then uses label propagation)
 bool cc_union_find(Graph &g, thv_stats *st);
-bool hint_trees_meet(Graph &g, hipStream_t s);
 void run_sssp(Graph &g, uint32_t src, uint32_t *out, thv_stats *st);
 void run_pr(Graph &g, int mode, float damping, float tol, int max_iter,
             float *out, thv_stats *st);
