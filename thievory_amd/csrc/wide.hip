@@ -471,8 +471,8 @@ static void number_destinations(Graph64 &g, const uint64_t *dst, const uint32_t 
   // writes a piece's records; how many of its destinations are missing
   auto number = [&](uint64_t e0, uint64_t cnt, bool final) {
     if (held != e0) {
-      HIPC(hipMemcpyAsync(d_dst, dst + e0, cnt * 8, hipMemcpyHostToDevice, s));
-      if (w) HIPC(hipMemcpyAsync(d_w, w + e0, cnt * 4, hipMemcpyHostToDevice, s));
+      HIPC(hipMemcpy(d_dst, dst + e0, cnt * 8, hipMemcpyHostToDevice));
+      if (w) HIPC(hipMemcpy(d_w, w + e0, cnt * 4, hipMemcpyHostToDevice));
       held = e0;
     }
     launch_fill_u32(reinterpret_cast<uint32_t *>(d_n), 0u, 2, s);
@@ -515,7 +515,7 @@ static void number_destinations(Graph64 &g, const uint64_t *dst, const uint32_t 
   for (uint64_t e0 = 0; e0 < g.m; e0 += piece)
     if (again[e0 / piece]) number(e0, std::min(piece, g.m - e0), true);
   g.h_extra.resize(x);
-  HIPC(hipMemcpyAsync(g.h_extra.data(), extra.p, x * 8, hipMemcpyDeviceToHost, s));
+  HIPC(hipMemcpy(g.h_extra.data(), extra.p, x * 8, hipMemcpyDeviceToHost));
   HIPC(hipStreamSynchronize(s));
   g.d_uid.swap(uid);
 }
@@ -820,13 +820,13 @@ void wide_gather(Graph64 &g, const uint64_t *at, uint64_t k, uint64_t *out) {
   DevMem &d = k <= KEEP ? g.at : own;
   if (d.bytes < k * 16) d.alloc(k * 16);
   uint64_t *d_at = d.as<uint64_t>(), *d_out = d_at + k;
-  HIPC(hipMemcpyAsync(d_at, at, k * 8, hipMemcpyHostToDevice, g.stream));
+  HIPC(hipMemcpy(d_at, at, k * 8, hipMemcpyHostToDevice));
   hipLaunchKernelGGL(k_wide_gather, dim3(grid_of(k, 16 * g.cus)), dim3(WBS), 0, g.stream,
                      g.val.as<uint64_t>(), g.d_uid.as<uint64_t>(), g.k, g.N,
                      g.last_algo == THV_ALGO_CC, g.n + 1, g.lone, d_at, k, d_out);
   HIPC(hipGetLastError());
-  HIPC(hipMemcpyAsync(out, d_out, k * 8, hipMemcpyDeviceToHost, g.stream));
   HIPC(hipStreamSynchronize(g.stream));
+  HIPC(hipMemcpy(out, d_out, k * 8, hipMemcpyDeviceToHost));
 }
 
 }  // namespace thv
