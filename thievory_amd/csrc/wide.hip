@@ -185,18 +185,23 @@ __device__ __forceinline__ bool flush_block(const WideArgs &a, ItemBuf &b, Block
   return found;
 }
 
-// Every listed vertex's segments (CC's first queue).
+// CC's first queue: every list's first segment in the order of the ids, so that
+// the least labels set out first (a random graph of degree 16 took a third
+// round, half as many edges again, whenever vertex 0 came late), then the
+// longer lists' other segments.  *nqn is k before.
 __global__ void __launch_bounds__(XBS) k_wide_all(WideArgs a) {
-  __shared__ uint64_t buf[XBS / 64][QBUF];
-  __shared__ BlockEnd end;
-  ItemBuf ib{buf[threadIdx.x >> 6], 0, false};
   const uint64_t T = (uint64_t)gridDim.x * XBS;
   for (uint64_t j = (uint64_t)blockIdx.x * XBS + threadIdx.x; j - lane_id() < a.k; j += T) {
-    const bool take[1] = {j < a.k};
-    const uint64_t w[1] = {j};
-    append(a, ib, take, w);
+    uint32_t more = 0;
+    if (j < a.k) {
+      a.nq[j] = j;
+      more = (uint32_t)((a.loff[j + 1] - a.loff[j] - 1) >> a.seg_shift);  // lists are not empty
+    }
+    if (!wave_ballot(more != 0)) continue;
+    const uint32_t inc = wave_incl_scan(more);
+    const uint64_t at = claim(a.nqn, (uint32_t)__builtin_amdgcn_readlane((int)inc, 63)) + inc - more;
+    for (uint32_t i = 0; i < more; i++) a.nq[at + i] = (uint64_t)(i + 1) << ITEM_BITS | j;
   }
-  flush_block(a, ib, end);
 }
 
 template <int ALGO, int REC>
@@ -279,7 +284,7 @@ __global__ void k_wide_end(unsigned long long *qn, const unsigned long long *nqn
 
 // The start of a run: every value `none` (CC: the vertex's id) but the
 // source's 1, no stamps, the counters clear; the queue holds the source's
-// segments (CC: nothing yet).
+// segments (CC: as many as there are lists, k_wide_all's).
 __global__ void __launch_bounds__(WBS)
 k_wide_init(WideArgs a, uint64_t N, bool ids, uint64_t src, unsigned long long *ctr,
             uint32_t nctr) {
@@ -293,6 +298,7 @@ k_wide_init(WideArgs a, uint64_t N, bool ids, uint64_t src, unsigned long long *
     for (uint32_t i = threadIdx.x; i < nctr; i += WBS) ctr[i] = 0;
     __threadfence();
     __syncthreads();
+    if (ids && threadIdx.x == 0) *a.nqn = a.k;
     if (threadIdx.x < 64 && src < a.k) {
       ItemBuf ib{buf, 0, false};
       const bool take[1] = {threadIdx.x == 0};
