@@ -276,6 +276,9 @@ int thv_pr(thv_graph *g, int mode, float damping, float tol, int max_iter,
  * thv_store_config (greedy runs of lists of at most partition_edges
  * records, densest in HBM up to the budget, the rest zero-copy); the
  * default is all in HBM with 2^16-record runs.  Traversal is top-down.
+ * Only vertices that a list names or belongs to take device memory, but a
+ * graph whose n x 8 bytes exceed the free device memory is THV_ENOMEM at its
+ * first algorithm call.
  * digest3 (nullable) receives the sum of mix64(mix64(v) + value) over the
  * vertices with a value other than n + 1 (mod 2^64; CC: over all), their
  * count and the largest value; out (nullable) the n values. */
@@ -302,7 +305,14 @@ void thv_graph64_close(thv_graph64 *g);
 
 /* Runs k <= 64 BFS (algo THV_ALGO_BFS) or SSSP (THV_ALGO_SSSP) queries in
  * one persistent launch sequence: per-vertex 64-bit source masks for BFS,
- * lane-packed distances for SSSP.  out_hash[k] receives the digest
+ * lane-packed distances for SSSP.  The engine (its device memory: about 64
+ * bytes per vertex for BFS, 56 + 4 k for SSSP) stays with the library when the
+ * call returns, for the next batch on the graph: at most one engine per graph
+ * and algorithm and 4 GiB in all, none for calls with out_full.  It is freed
+ * when the graph is closed or its store changes, before a server is started,
+ * when one of the library's allocations fails, and by thv_device_memory;
+ * another allocator in the process can call that to have the memory back.
+ * out_hash[k] receives the digest
  *   sum over v with out[v] != n+1 of mix64((v << 32) | out[v])  (mod 2^64)
  * where mix64 is the SplitMix64 output function, out_reached[k] the reached
  * counts, out_depth[k] the largest finite value.  out_full (nullable) gets
@@ -415,7 +425,8 @@ int thv_device_info(char *name, size_t name_len, int *cus,
  * HBM, out[3] a device -> device copy (bytes read + written); all GB/s. */
 int thv_link_probe(uint64_t bytes, double *out4);
 
-/* Free and total device memory (hipMemGetInfo). */
+/* Free and total device memory (hipMemGetInfo), after the engines kept from
+ * finished batches (thv_batch) have been freed: what any caller can have. */
 int thv_device_memory(uint64_t *free_bytes, uint64_t *total_bytes);
 
 #ifdef __cplusplus

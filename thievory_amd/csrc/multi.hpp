@@ -54,15 +54,17 @@ struct MultiEngine {
   uint64_t pend_finish = 0;    // SSSP lanes done, digest pending
   uint64_t pend_clear = 0;     // BFS lanes done, seen bits to clear before an admission
   bool finish_last = false;    // digest the finished SSSP lanes in one pass, at the end
+                               // (a batch; a server wants each as soon as it is done)
   // SSSP levels with a grid of ROOM_BPC blocks a CU, of the 7 that fit: the
   // kernels of BFS levels on other streams find registers and LDS at once,
   // where they waited for a whole SSSP level.  50/50 stream at 394 queries/s on
   // R-MAT 25, BFS p50 / SSSP p50 / saturated throughput, with a block a chunk
-  // 119 ms / 85 ms / 813 a second; with 4 a CU 4 / 124 / 662, 5 7 / 114 / 728,
-  // 6 24 / 104 / 740.
+  // 119 ms / 85 ms / 813 a second; with 4 a CU 4 / 124 / 662, 5 7 / 114 / 728 (in
+  // another run 8 / 115 / 762), 6 24 / 104 / 740.  Where few queries are BFS the
+  // room costs SSSP throughput: with 2% of them, R-MAT 20, 5% saturated with 30%
+  // of the edges in HBM, 11% with all (BFS p50 at 60% load 2.1 and 0.3 ms).
   static constexpr uint32_t ROOM_BPC = 5;
   bool leave_room = false;
-                               // (a batch; a server wants each as soon as it is done)
   uint64_t finalizing = 0;     // lanes whose digest is in flight this level
   uint32_t voff[MAXL] = {};
   uint32_t last_val[MAXL] = {};

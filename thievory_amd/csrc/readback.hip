@@ -3,7 +3,11 @@
 // hipMemcpy into pageable memory moves about 18 GB/s here; writes into pinned
 // memory 56.  So a large array goes through a ring of pinned slots: a kernel
 // fills one slot while worker threads copy the others out, each its own
-// slice of every slot.
+// slice of every slot.  The threads watch the flags, so a copy takes more of the
+// host than hipMemcpy did and less time: CC on R-MAT 23 with 1 / 2 / 4 / 8 callers
+// at once, each with a graph, 1.04 / 0.85 / 0.79 / 0.91 ms a call (3.57 / 2.08 /
+// 2.08 / 2.09) for 6.2 / 6.7 / 10.2 / 12.4 ms of CPU time (3.6 - 3.9); on two
+// CPUs 1.3 / 1.4 / 1.5 / 1.7 ms.
 #include <algorithm>
 #include <atomic>
 #include <mutex>

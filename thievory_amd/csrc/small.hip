@@ -17,9 +17,9 @@
 //   3. the returning atomic on the destination (visited bit or value); the
 //      winners append to the queue, one LDS atomic per wave.
 // Bound: the latency of those rounds, about 0.8 us each: a 2,001-vertex path
-// behind a 19,999-leaf star takes 5.3 ms (2.6 us a level) against 108 ms by
+// behind a 19,999-leaf star takes 5.4 ms (2.7 us a level) against 109 ms by
 // the general path, SSSP on a 500 x 500 grid (2,260 rounds, and as many
-// buckets again) 12.2 ms against 133.
+// buckets again) 13.3 ms against 174.
 //
 // The block gives up (and the general path takes over) when a frontier has
 // more than SPARSE_MAX vertices (its LDS holds 24 bytes of each) or SMALL_EDGES
