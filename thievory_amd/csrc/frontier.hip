@@ -566,8 +566,11 @@ __global__ void __launch_bounds__(CBS, 4) k_bu_probe(ProbeArgs a) {
       const int src = (int)(2 * r + (lane >> 5));
       const uint32_t bit = 1u << (lane & 31);
       const bool in = r * 64 + lane < nin;
-      if (in && !((uint32_t)__shfl((int)vw, src, 64) & bit)) un |= 1u << r;
-      if ((uint32_t)__shfl((int)rw, src, 64) & bit) dev |= 1u << r;
+      // (every lane takes part: the words' lanes may hold no vertex of the round)
+      const uint32_t vr = (uint32_t)__shfl((int)vw, src, 64);
+      const uint32_t rr = (uint32_t)__shfl((int)rw, src, 64);
+      if (in && !(vr & bit)) un |= 1u << r;
+      if (rr & bit) dev |= 1u << r;
     }
     nun += __popc(un);
     uint32_t m = 0;  // hits of word `lane` (lanes 0-31)
