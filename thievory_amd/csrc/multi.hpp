@@ -60,9 +60,10 @@ struct MultiEngine {
   // where they waited for a whole SSSP level.  50/50 stream at 394 queries/s on
   // R-MAT 25, BFS p50 / SSSP p50 / saturated throughput, with a block a chunk
   // 119 ms / 85 ms / 813 a second; with 4 a CU 4 / 124 / 662, 5 7 / 114 / 728 (in
-  // another run 8 / 115 / 762), 6 24 / 104 / 740.  Where few queries are BFS the
-  // room costs SSSP throughput: with 2% of them, R-MAT 20, 5% saturated with 30%
-  // of the edges in HBM, 11% with all (BFS p50 at 60% load 2.1 and 0.3 ms).
+  // another run 8 / 115 / 762), 6 24 / 104 / 740.  On R-MAT 20 with 30% of the
+  // edges in HBM, a block a chunk / 5 a CU: 2% BFS queries, saturated 4,880 /
+  // 4,775 a second and BFS p50 at 3,000 2.1 / 0.3 ms; 50/50 at 5,000 BFS 7.9 /
+  // 3.9 ms, SSSP 21 / 42.
   static constexpr uint32_t ROOM_BPC = 5;
   bool leave_room = false;
   uint64_t finalizing = 0;     // lanes whose digest is in flight this level

@@ -48,7 +48,7 @@ struct SmallShared {
   uint32_t nval[QCAP];          // VAL: the values they were queued with
   unsigned long long part[SB / 64];
   unsigned long long sum[12];
-  uint32_t cnt, over, fars, lo, any;
+  uint32_t cnt, over, fars, lo;
 };
 
 // One thread's vertices and edges of the frontier left in the bitmap (host,
