@@ -1159,7 +1159,11 @@ void MultiEngine::launch_top_down(LevelCtr *c, uint64_t lanes) {
       const bool large = h.qw[0] + h.qw[1] >= 8ull * g.cus * SSSP_LARGE;
       const uint32_t C = large ? SSSP_LARGE : SSSP_C;
       const uint64_t chunks = div_up(h.qw[0], C) + div_up(h.qw[1], C);
-      const uint64_t most = leave_room ? (uint64_t)ROOM_BPC * g.cus : 1u << 30;
+      // (a level's time: its host records at the link's rate, some 50 ps a record)
+      const double ms = (double)h.qw[0] * 8 / (g.do_link_gbps * 1e6) +
+                        (double)(h.qw[0] + h.qw[1]) * 50e-9;
+      const bool room = leave_room && ms >= ROOM_MS;
+      const uint64_t most = room ? (uint64_t)ROOM_BPC * g.cus : 1u << 30;
       const uint64_t sg = std::max<uint64_t>(1, std::min<uint64_t>(chunks, most));
       if (large) launch_sssp<SSSP_LARGE>(a, (uint32_t)sg, stream);
       else launch_sssp<SSSP_C>(a, (uint32_t)sg, stream);

@@ -55,15 +55,21 @@ struct MultiEngine {
   uint64_t pend_clear = 0;     // BFS lanes done, seen bits to clear before an admission
   bool finish_last = false;    // digest the finished SSSP lanes in one pass, at the end
                                // (a batch; a server wants each as soon as it is done)
-  // SSSP levels with a grid of ROOM_BPC blocks a CU, of the 7 that fit: the
-  // kernels of BFS levels on other streams find registers and LDS at once,
-  // where they waited for a whole SSSP level.  50/50 stream at 394 queries/s on
-  // R-MAT 25, BFS p50 / SSSP p50 / saturated throughput, with a block a chunk
-  // 119 ms / 85 ms / 813 a second; with 4 a CU 4 / 124 / 662, 5 7 / 114 / 728 (in
-  // another run 8 / 115 / 762), 6 24 / 104 / 740.  On R-MAT 20 with 30% of the
-  // edges in HBM, a block a chunk / 5 a CU: 2% BFS queries, saturated 4,880 /
-  // 4,775 a second and BFS p50 at 3,000 2.1 / 0.3 ms; 50/50 at 5,000 BFS 7.9 /
-  // 3.9 ms, SSSP 21 / 42.
+  // SSSP levels of ROOM_MS or more with a grid of ROOM_BPC blocks a CU, of the
+  // 7 that fit: the kernels of BFS levels on other streams find registers and LDS
+  // at once, where they waited for a whole SSSP level.  50/50 stream at 394
+  // queries/s on R-MAT 25, BFS p50 / SSSP p50 / saturated throughput, with a block
+  // a chunk 119 ms / 85 ms / 813 a second; with 4 a CU 4 / 124 / 662, 5 7 / 114 /
+  // 728 (in another run 8 / 115 / 762), 6 24 / 104 / 740.  In shorter levels BFS
+  // waits less, and room costs throughput or SSSP more than that gives.  50/50
+  // streams, room in all levels / from 3 ms / in none, queries a second saturated,
+  // then p50 of BFS and of SSSP at 40 to 60% of that:
+  //   R-MAT 18  48,900 / 53,000 / 52,000   1.1 / 1.4 / 1.4    4.9 / 4.3 / 4.4 ms
+  //   20        19,400 / 21,300 / 21,500   1.1 / 2.4 / 2.5   10.5 / 9.4 / 9.3
+  //   20, 30% in HBM  8,260 / 8,390 / 8,330   3.8 / 7.9 / 7.4   34 / 19 / 19
+  //   23         2,990 / 3,040 / 3,490     2.2 / 1.9 / 17      27 / 28 / 21
+  //   23, 30%    1,020 / 1,010 / 1,070     6.8 / 6.0 / 41     113 / 109 / 104
+  static constexpr double ROOM_MS = 3.0;
   static constexpr uint32_t ROOM_BPC = 5;
   bool leave_room = false;
   uint64_t finalizing = 0;     // lanes whose digest is in flight this level

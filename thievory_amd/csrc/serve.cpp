@@ -63,7 +63,7 @@ struct Server {
   // saturated at R-MAT 25).
   static constexpr int COHORT_ENGINES = 4;
   static constexpr double SPILL_MS = 10.0;
-  // SSSP levels leave room (MultiEngine::leave_room) while BFS queries come:
+  // Long SSSP levels leave room (MultiEngine::leave_room) while BFS queries come:
   // one may arrive during a level that was launched with none waiting
   static constexpr double BFS_RECENT_MS = 1000.0;
   double last_bfs = -2 * BFS_RECENT_MS;
